@@ -97,6 +97,13 @@ size_t sqa_workspace_bytes(int batch, int q_len, int num_query_heads, int num_kv
  * 4-byte (SQA_ERR_INVALID otherwise), and a plan's partial sums must stay within
  * 0xFFFF0000 bytes (SQA_ERR_INVALID; the automatic plans need a few MB to ~40 MB).
  * Allocates nothing and never synchronises.
+ * A fixed plan (pages_per_split > 0) says which pages are read: the first
+ * num_splits * pages_per_split of every sequence. Where the given workspace also
+ * holds the automatic plan over those pages and that plan is the faster cut, the
+ * call runs it instead (the sums then round in another order; the same arguments
+ * and workspace size give the same bits). A workspace of that size, that is the
+ * larger of sqa_workspace_bytes for the two plans, lets a few sequences in coarse
+ * chunks use the whole chip; one of the fixed plan's own size is always enough.
  * `timing_events`: NULL, or an array of 3 hipEvent_t recorded on `stream`
  * before the partial kernel, between the two kernels and after the merge
  * kernel (used by the benchmark to time the partial kernel alone).

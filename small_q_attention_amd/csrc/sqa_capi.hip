@@ -4,6 +4,8 @@
 #include "sqa.h"
 #include "sqa_internal.h"
 
+#include <algorithm>
+
 #include <math.h>
 #include <stdarg.h>
 #include <stddef.h>
@@ -40,6 +42,125 @@ std::mutex g_cu_mutex;
 std::vector<int> g_cu_count;  // cached per device
 
 long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
+
+// Splits of `pps` pages (held to the sequence and to kMaxSplitPages) over `pages`.
+int fixed_plan(int batch, int num_kv_heads, long long pages, long long pps, int* num_splits,
+               int* pages_per_split) {
+  if (pps > pages) pps = pages;
+  if (pps > sqa::kMaxSplitPages) pps = sqa::kMaxSplitPages;
+  if (pps < 1) pps = 1;
+  long long splits = ceil_div(pages, pps);
+  if (splits < 1) splits = 1;
+  if ((long long)batch * num_kv_heads * splits > 0x7fffffffLL)
+    return fail(SQA_ERR_INVALID, "grid too large");
+  *num_splits = (int)splits;
+  *pages_per_split = (int)pps;
+  return SQA_OK;
+}
+
+// The automatic plan (sqa_plan_splits with chunk_keys 0) over `pages` pages per
+// sequence; `known`: no sequence spans more.
+int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int head_dim,
+                   long long pages, int max_pages, bool known, int* num_splits,
+                   int* pages_per_split) {
+  int cus = sqa_device_cu_count(device);
+  if (cus <= 0) return SQA_ERR_HIP;
+  // One wave of resident workgroups over the whole chip.
+  const sqa::LaunchShape sh = sqa::launch_shape((int)rows, num_kv_heads, head_dim);
+  const long long head_groups = (num_kv_heads + sh.heads - 1) / sh.heads;
+  const long long slots_target = ceil_div((long long)cus * sh.wg_per_cu, head_groups);
+  if (batch > 1 && batch <= sqa::kMaxBalancedBatch) {
+    // Balanced plan: the kernel sizes splits from the batch's total pages,
+    // so ragged batches keep every workgroup equally busy. The slot count
+    // leaves one spare slot per sequence (rounding up each sequence's last
+    // split) and keeps a split within kMaxSplitPages pages.
+    long long target = slots_target;
+    const long long cap = ceil_div((long long)batch * max_pages, sqa::kMaxSplitPages);
+    if (target < cap) target = cap;
+    if ((target + batch) * num_kv_heads > 0x7fffffffLL)
+      return fail(SQA_ERR_INVALID, "grid too large");
+    *num_splits = (int)(target + batch);
+    // With a known max_seq_len the kernels first assume every sequence spans
+    // that many pages (and check it): -pages.
+    *pages_per_split = known ? -(int)pages : 0;
+    return SQA_OK;
+  }
+  const long long splits = ceil_div(slots_target, batch);
+  long long pps = ceil_div(pages, splits);
+  // Each split leaves a partial row per query row for the merge. Past 32
+  // rows (the 64-row kernel), sequences of more than 64 four-page splits
+  // start at 8 pages: there the merge of the extra splits costs more than the
+  // shorter splits save (one sequence, KV 8K, q16, per call: 23.9 us at 64 x
+  // 8 pages, 26.7 at 128 x 4), while shorter ones gain from 4. Up to 32 rows
+  // 4-page pieces take the register ring in one softmax step, and 4 pages win
+  // (KV 8K, q8: 18.0 us at 128 x 4, 19.0 at 64 x 8).
+  const long long min_pps = rows > 32 && pages > 64 * sqa::kMinSplitPages
+                                ? 2 * sqa::kMinSplitPages
+                                : sqa::kMinSplitPages;
+  if (pps < min_pps) pps = min_pps;
+  return fixed_plan(batch, num_kv_heads, pages, pps, num_splits, pages_per_split);
+}
+
+// What a call with a fixed plan runs. The plan says which pages of every
+// sequence are read (the first num_splits * pages_per_split); how they are cut
+// changes only the order of the sums. Chunks of a caller's choosing (the
+// reference's default is 512 keys) leave most of the chip idle for a few
+// sequences (one of 8K keys: 32 workgroups on 256 CUs) and run a second,
+// partly filled wave of workgroups for many. So the same pages are cut as the
+// automatic plan cuts them, where the caller's workspace holds that plan:
+// *num_splits and *pages_per_split are replaced, and the pages a sequence may
+// span returned (kernel_pages unchanged without a re-cut).
+//
+// Measured with 512-key chunks, as given -> re-cut (us per call, back to back):
+// one sequence of 8K keys 35.2 -> 13.7 (q_len 2), of 32K keys 46.1 -> 28.4; two
+// of 8K keys, q_len 8, 43.6 -> 23.9. Kept as given:
+// - plans past kMaxBalancedBatch sequences (the automatic plan is then another
+//   fixed one);
+// - several sequences whose splits come to more than a quarter of a wave of
+//   work items (an eighth past 32 rows) and less than four waves: there a balanced item that spans a
+//   sequence end costs as much as the idle workgroups (64 ragged sequences of
+//   up to 1K keys, q_len 8: 49 as given, 68 re-cut), while four waves of
+//   start-ups cost 4-70%;
+// - one split per sequence (no partials, no merge kernel) unless an item gets
+//   shorter by kMinPagesSaved pages, and, for several sequences, by twice that
+//   with at most 1/16 of a wave of items (200 keys, 8 sequences: 15 us as given,
+//   17 re-cut; 512 keys: 32 and 15).
+constexpr int kMinPagesSaved = 12;
+long long recut_plan(const sqa_attention_args& a, long long rows, long long kernel_pages,
+                     int* num_splits, int* pages_per_split) {
+  if (sqa::is_balanced(*pages_per_split) || a.batch > sqa::kMaxBalancedBatch || !a.workspace ||
+      (uintptr_t)a.workspace % 16)
+    return kernel_pages;
+  const long long cover = std::min((long long)*num_splits * *pages_per_split, kernel_pages);
+  if (cover >= (1LL << 24) || a.batch * cover >= (1LL << 30)) return kernel_pages;
+  int device = -1, ns = 0, pps = 0;
+  if (hipGetDevice(&device) != hipSuccess ||
+      automatic_plan(device, a.batch, rows, a.num_kv_heads, a.head_dim, cover, (int)cover, true,
+                     &ns, &pps) != SQA_OK)
+    return kernel_pages;
+  const long long item = sqa::is_balanced(pps)
+                             ? sqa::packed_item_pages((int)(a.batch * cover), ns - a.batch)
+                             : pps;
+  const long long given = (long long)a.batch * *num_splits;
+  if (a.batch > 1) {
+    const long long wave = ns - a.batch;  // items of the balanced plan
+    if (*num_splits > 1 ? (rows > 32 ? 8 : 4) * given > wave && given < 4 * wave
+                        : 16 * given > wave)
+      return kernel_pages;
+  }
+  if (*num_splits == 1 && cover - item < (a.batch > 1 ? 2 : 1) * kMinPagesSaved)
+    return kernel_pages;
+  const unsigned long long part_o_bytes =
+      (unsigned long long)sqa::plan_slots(a.batch, ns, pps) * a.num_kv_heads * rows * a.head_dim *
+      sizeof(float);
+  if (part_o_bytes > sqa::kMaxPartialBytes ||
+      sqa_workspace_bytes(a.batch, a.q_len, a.num_query_heads, a.num_kv_heads, a.head_dim, ns,
+                          pps) > a.workspace_bytes)
+    return kernel_pages;
+  *num_splits = ns;
+  *pages_per_split = pps;
+  return cover;
+}
 
 }  // namespace
 
@@ -87,58 +208,12 @@ int sqa_plan_splits(int device, int batch, int q_len, int num_query_heads, int n
     const long long need = ceil_div(max_seq_len, sqa::kPageSize);
     pages = need < pages ? need : pages;
   }
-  long long pps;
-  if (chunk_keys > 0) {
-    pps = ceil_div(chunk_keys, sqa::kPageSize);
-  } else {
-    int cus = sqa_device_cu_count(device);
-    if (cus <= 0) return SQA_ERR_HIP;
-    // One wave of resident workgroups over the whole chip.
-    const sqa::LaunchShape sh =
-        sqa::launch_shape(q_len * (num_query_heads / num_kv_heads), num_kv_heads, head_dim);
-    const long long head_groups = (num_kv_heads + sh.heads - 1) / sh.heads;
-    const long long slots_target = ceil_div((long long)cus * sh.wg_per_cu, head_groups);
-    if (batch > 1 && batch <= sqa::kMaxBalancedBatch) {
-      // Balanced plan: the kernel sizes splits from the batch's total pages,
-      // so ragged batches keep every workgroup equally busy. The slot count
-      // leaves one spare slot per sequence (rounding up each sequence's last
-      // split) and keeps a split within kMaxSplitPages pages.
-      long long target = slots_target;
-      const long long cap = ceil_div((long long)batch * max_pages, sqa::kMaxSplitPages);
-      if (target < cap) target = cap;
-      if ((target + batch) * num_kv_heads > 0x7fffffffLL)
-        return fail(SQA_ERR_INVALID, "grid too large");
-      *num_splits = (int)(target + batch);
-      // With a known max_seq_len the kernels first assume every sequence spans
-      // that many pages (and check it): -pages.
-      *pages_per_split = max_seq_len > 0 ? -(int)pages : 0;
-      return SQA_OK;
-    }
-    const long long splits = ceil_div(slots_target, batch);
-    pps = ceil_div(pages, splits);
-    // Each split leaves a partial row per query row for the merge. Past 32
-    // rows (the 64-row kernel), sequences of more than 64 four-page splits
-    // start at 8 pages: there the merge of the extra splits costs more than the
-    // shorter splits save (one sequence, KV 8K, q16, per call: 23.9 us at 64 x
-    // 8 pages, 26.7 at 128 x 4), while shorter ones gain from 4. Up to 32 rows
-    // 4-page pieces take the register ring in one softmax step, and 4 pages win
-    // (KV 8K, q8: 18.0 us at 128 x 4, 19.0 at 64 x 8).
-    const bool past32 = (long long)q_len * (num_query_heads / num_kv_heads) > 32;
-    const long long min_pps = past32 && pages > 64 * sqa::kMinSplitPages
-                                  ? 2 * sqa::kMinSplitPages
-                                  : sqa::kMinSplitPages;
-    if (pps < min_pps) pps = min_pps;
-  }
-  if (pps > pages) pps = pages;
-  if (pps > sqa::kMaxSplitPages) pps = sqa::kMaxSplitPages;
-  if (pps < 1) pps = 1;
-  long long splits = ceil_div(pages, pps);
-  if (splits < 1) splits = 1;
-  if ((long long)batch * num_kv_heads * splits > 0x7fffffffLL)
-    return fail(SQA_ERR_INVALID, "grid too large");
-  *num_splits = (int)splits;
-  *pages_per_split = (int)pps;
-  return SQA_OK;
+  if (chunk_keys == 0)
+    return automatic_plan(device, batch, (long long)q_len * (num_query_heads / num_kv_heads),
+                          num_kv_heads, head_dim, pages, max_pages, max_seq_len > 0, num_splits,
+                          pages_per_split);
+  return fixed_plan(batch, num_kv_heads, pages, ceil_div(chunk_keys, sqa::kPageSize), num_splits,
+                    pages_per_split);
 }
 
 size_t sqa_workspace_bytes(int batch, int q_len, int num_query_heads, int num_kv_heads,
@@ -170,8 +245,8 @@ namespace {
 int run_attention(const sqa_attention_args& a) {
   const int batch = a.batch, q_len = a.q_len, num_query_heads = a.num_query_heads;
   const int num_kv_heads = a.num_kv_heads, head_dim = a.head_dim, page_size = a.page_size;
-  const int max_pages = a.max_pages, num_splits = a.num_splits;
-  const int pages_per_split = a.pages_per_split;
+  const int max_pages = a.max_pages;
+  int num_splits = a.num_splits, pages_per_split = a.pages_per_split;
   const int64_t num_pages = a.kv.num_pages;
   if (!a.query || !a.kv.k || !a.kv.v || !a.block_tables || !a.seq_lens || !a.output)
     return fail(SQA_ERR_INVALID, "null tensor pointer");
@@ -235,8 +310,8 @@ int run_attention(const sqa_attention_args& a) {
   if (pages_per_split > sqa::kMaxSplitPages)
     return fail(SQA_ERR_INVALID, "pages_per_split %d exceeds %d", pages_per_split,
                 sqa::kMaxSplitPages);
-  const bool balanced = sqa::is_balanced(pages_per_split);
-  const int spec_pages = sqa::spec_pages_of(pages_per_split);
+  bool balanced = sqa::is_balanced(pages_per_split);
+  int spec_pages = sqa::spec_pages_of(pages_per_split);
   if (balanced) {
     // pages_per_split <= 0 selects the balanced plan (sqa_plan_splits); -P expects
     // P pages in every sequence.
@@ -272,12 +347,18 @@ int run_attention(const sqa_attention_args& a) {
     return fail(SQA_ERR_WORKSPACE, "workspace must be 16-byte aligned");
 
   // fp16 outputs keep fp16 partial rows (half of the region), bf16 fp32 ones.
-  const unsigned long long part_o_bytes =
-      (unsigned long long)sqa::plan_slots(batch, num_splits, pages_per_split) * num_kv_heads *
-      rows * head_dim * (a.dtype == SQA_DTYPE_F16 ? 2 : 4);
+  const auto partial_bytes = [&] {
+    return (unsigned long long)sqa::plan_slots(batch, num_splits, pages_per_split) *
+           num_kv_heads * rows * head_dim * (a.dtype == SQA_DTYPE_F16 ? 2 : 4);
+  };
+  unsigned long long part_o_bytes = partial_bytes();
   if ((balanced || num_splits > 1) && part_o_bytes > sqa::kMaxPartialBytes)
     return fail(SQA_ERR_INVALID, "the plan's partials (%llu bytes) exceed %llu bytes",
                 part_o_bytes, sqa::kMaxPartialBytes);
+  const long long call_pages = recut_plan(a, rows, kernel_pages, &num_splits, &pages_per_split);
+  balanced = sqa::is_balanced(pages_per_split);
+  spec_pages = sqa::spec_pages_of(pages_per_split);
+  part_o_bytes = partial_bytes();
   hipStream_t s = (hipStream_t)a.stream;
   hipEvent_t* ev = (hipEvent_t*)a.timing_events;
   void* workspace = a.workspace;
@@ -312,7 +393,7 @@ int run_attention(const sqa_attention_args& a) {
   pa.head_dim = head_dim;
   pa.bt_stride = max_pages;
   pa.page_shift = page_shift;
-  pa.max_pages = (int)kernel_pages;
+  pa.max_pages = (int)call_pages;
   pa.pages_per_split = balanced ? 0 : pages_per_split;
   pa.num_splits = num_splits;
   pa.spec_pages = spec_pages;
@@ -390,7 +471,7 @@ int run_attention(const sqa_attention_args& a) {
     ma.group = group;
     ma.rows = (int)rows;
     ma.head_dim = head_dim;
-    ma.max_pages = (int)kernel_pages;
+    ma.max_pages = (int)call_pages;
     ma.pages_per_split = pa.pages_per_split;
     ma.num_splits = num_splits;
     ma.spec_pages = spec_pages;
@@ -533,7 +614,7 @@ int sqa_paged_mtp_attention_noalloc(const void* query, const void* key_cache,
                                   batch, q_len, num_query_heads, num_kv_heads, head_dim, num_pages,
                                   page_size, max_pages, num_splits, pages_per_split, stream);
   a.workspace = ws;
-  a.workspace_bytes = ws ? kScratchBytes : 0;
+  a.workspace_bytes = need;  // what the plan needs: cut as a caller's workspace of that size is
   return run_attention(a);
 }
 
