@@ -225,6 +225,7 @@ template <int HD>
 struct KvNative {  // the query's 16-bit type
   static constexpr int kBytes = 2;
   static constexpr int KK = Dims<HD>::KK, VW = Dims<HD>::VW;
+  static constexpr int kLoads = KK + 4 * (VW > 4 ? VW / 4 : 1);  // instructions per page
   // One 16-byte load per fragment: dims 32*kk + 8*g.
   static __device__ __forceinline__ int q_dims(int kk, int g) { return 32 * kk + 8 * g; }
   static __device__ __forceinline__ unsigned k_lane_bytes(int g) { return 16 * g; }
@@ -274,6 +275,7 @@ template <int HD>
 struct KvFp8 {  // OCP e4m3 bytes, widened exactly to the query's type
   static constexpr int kBytes = 1;
   static constexpr int KK = Dims<HD>::KK, VW = Dims<HD>::VW;
+  static constexpr int kLoads = KK / 2 + 4;  // instructions per page
   // K rows are HD bytes: 16-byte loads per lane (64 bytes of a row per
   // instruction, as for the 16-bit types; 8-byte loads used 32 bytes per row
   // request and ran at 58% of peak instead of 78%). Load i holds dims
@@ -550,13 +552,17 @@ __device__ __forceinline__ void page_pv(WaveState<NB, HD>& st, const f4 (&s)[NB]
   }
 }
 
-template <int NB, int HD, typename E, typename KV, int HPW>
+// bits.get(dbits): the draft bits of the lane's rows, asked for on masked pages only.
+template <int NB, int HD, typename E, typename KV, int HPW, typename Bits>
 __device__ __forceinline__ void page_finish(WaveState<NB, HD>& st, f4 (&s)[NB],
-                                            PageV<HD, HPW>& pv, bool upper,
-                                            const unsigned long long (&dbits)[NB],
+                                            PageV<HD, HPW>& pv, bool upper, const Bits& bits,
                                             int draft_base, int tok0, int len, bool masked,
                                             float c) {
-  if (masked) mask_page<NB, HD, HPW>(s, pv, dbits, draft_base, tok0, len);
+  if (masked) {
+    unsigned long long dbits[NB];
+    bits.get(dbits);
+    mask_page<NB, HD, HPW>(s, pv, dbits, draft_base, tok0, len);
+  }
   float lm[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) lm[nb] = max4(s[nb]) * c;
@@ -576,12 +582,11 @@ __device__ __forceinline__ void page_finish(WaveState<NB, HD>& st, f4 (&s)[NB],
 // page p + 1 is past the piece (its slot holds a zero page); its scores become
 // -inf. Same sums as two page_finish steps up to fp32 rounding and the point
 // at which the lagging max is raised.
-template <int NB>
+template <int NB, typename Bits>
 __device__ __forceinline__ void pair_finish(WaveState<NB, 128>& st, f4 (&s0)[NB], f4 (&s1)[NB],
                                             KvFp8<128>::Regs r0, KvFp8<128>::Regs r1,
-                                            bool have1, const unsigned long long (&dbits)[NB],
-                                            int draft_base, int tok0, int len, bool masked,
-                                            float c) {
+                                            bool have1, const Bits& bits, int draft_base,
+                                            int tok0, int len, bool masked, float c) {
   using E = ElemF16;
   constexpr int MB = Dims<128>::MB;
   // Both conditions are uniform over the wave and rare (pages at the draft
@@ -589,6 +594,8 @@ __device__ __forceinline__ void pair_finish(WaveState<NB, 128>& st, f4 (&s0)[NB]
   // branch keeps their selects out of the common step.
   if (masked || !have1) {
     if (masked) {
+      unsigned long long dbits[NB];
+      bits.get(dbits);
       mask_scores<NB>(s0, dbits, draft_base, tok0, len);
       mask_scores<NB>(s1, dbits, draft_base, tok0 + kPageSize, len);
 #pragma unroll
@@ -690,13 +697,21 @@ struct ItemRange {
   int paired;   // a paired item of the expected-page plan (its loop time is timed)
 };
 
+// A value every lane needs from memory no workgroup of the call writes, at an
+// address the same in every lane: read through the scalar cache into a scalar
+// register (the compiler picks the vector path for plain loads here: it cannot see
+// that nothing writes there), without a place in the vector loads' order.
+__device__ __forceinline__ int scalar_load(const int32_t* p) {
+  return *(const __attribute__((address_space(4))) int32_t*)p;
+}
+
 // Fixed plan: sequence b owns slots b * num_splits + s.
 __device__ __forceinline__ ItemRange fixed_item(const PartialArgs& a, int item) {
   ItemRange r;
   r.b = item / a.num_splits;
   r.split = item - r.b * a.num_splits;
   r.p_begin = r.split * a.pages_per_split;
-  r.len = max(a.seq_lens[r.b], 0);
+  r.len = max(scalar_load(a.seq_lens + r.b), 0);
   const int pages = min((r.len + kPageSize - 1) / kPageSize, a.max_pages);
   r.p_end = min(r.p_begin + a.pages_per_split, pages);
   r.n_valid = min((pages + a.pages_per_split - 1) / a.pages_per_split, a.num_splits);
@@ -921,135 +936,167 @@ struct WaveRows {
   }
 };
 
-// Runs `piece(range, first_id)` for every piece of workgroup item `item`, with
-// the ids of the piece's first D pages loaded (index clamped into the
-// block-table row; ids past the piece are never used). Fixed plan: one piece
-// whose page range follows from `item` alone, so its ids are issued before the
-// sequence length is read and both arrive in one round trip. Balanced plan:
-// all lengths, the packed plan's wave reductions, then each piece's ids; with
-// an expected page count (every sequence spec_pages pages, item size spec_pps
-// from the host) the plan needs no lengths, so the first piece's ids go out
-// with them, and a length that does not match falls back to the plan from the
-// loaded lengths. Piece fields are the same in every lane (readfirstlane): the
-// piece, and the buffer-resource addresses built from it, stay in scalar
-// registers. Consecutive pieces are separated by a barrier (they reuse the
-// workgroup's LDS). Returns whether the item ran as a paired item (every
-// workgroup of a call returns the same).
+// The same in every lane (readfirstlane tells the compiler): the piece, and the
+// buffer-resource addresses built from it, stay in scalar registers.
+__device__ __forceinline__ void make_uniform(ItemRange& it) {
+  it.b = __builtin_amdgcn_readfirstlane(it.b);
+  it.split = __builtin_amdgcn_readfirstlane(it.split);
+  it.p_begin = __builtin_amdgcn_readfirstlane(it.p_begin);
+  it.p_end = __builtin_amdgcn_readfirstlane(it.p_end);
+  it.len = __builtin_amdgcn_readfirstlane(it.len);
+  it.n_valid = __builtin_amdgcn_readfirstlane(it.n_valid);
+  it.slot0 = __builtin_amdgcn_readfirstlane(it.slot0);
+  it.g_end = __builtin_amdgcn_readfirstlane(it.g_end);
+}
+
+// A work item on its way through its pieces: a fixed plan has one (g 0, g_end 1),
+// a balanced item the pieces packed_piece() finds from global page g to g_end.
+struct ItemWalk {
+  PackedBatch pb;
+  ItemRange it;     // the current piece
+  int g_end;        // balanced: where the item's pages end
+  int item_end;     // balanced: where the item ends
+  bool paired;      // the item runs as a paired item
+};
+
+template <int D>
+__device__ __forceinline__ void load_first_ids(const PartialArgs& a, int seq, int p0,
+                                               int (&first_id)[D]) {
+  const int32_t* row = a.block_tables + (size_t)max(seq, 0) * a.bt_stride;
+#pragma unroll
+  for (int j = 0; j < D; ++j)
+    first_id[j] = scalar_load(row + (min(max(p0 + j, 0), a.max_pages - 1) >> a.page_shift));
+}
+
+// A balanced item's piece from global page g on; false if the item has none there.
+// A piece has a sequence and at least one page unless the item ends in the gap
+// before a sequence start (no further pieces then); the check also keeps every
+// walk finite whatever the inputs.
+__device__ __forceinline__ bool piece_at(const PartialArgs& a, ItemWalk& w, int item, int g) {
+  if (g >= w.g_end) return false;  // uniform
+  w.it = packed_piece(a, w.pb, item, g, w.item_end);
+  make_uniform(w.it);
+  w.it.paired = w.paired;
+  return w.it.b >= 0 && w.it.p_end > w.it.p_begin;
+}
+
+// Finds the first piece of workgroup item `item` and loads the ids of its first D
+// pages (index clamped into the block-table row; ids past the piece are never
+// used); false if the item has no piece. Fixed plan: one piece whose page range
+// follows from `item` alone, so its ids are issued before the sequence length is
+// read and both arrive in one round trip. Balanced plan: all lengths, the packed
+// plan's wave reductions, then the ids; with an expected page count (every
+// sequence spec_pages pages, item size spec_pps from the host) the plan needs no
+// lengths, so the ids go out with them, and a length that does not match falls
+// back to the plan from the loaded lengths.
+// kPairs: paired items may be asked for.
+template <int D, bool kPairs>
+__device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView& v, int item,
+                                            ItemWalk& w, int (&first_id)[D]) {
+  const int lane = threadIdx.x & 63;
+  PackedBatch& pb = w.pb;
+  w.paired = false;
+  if (!is_balanced(a.pages_per_split)) {
+    const int seq = item / a.num_splits;
+    load_first_ids<D>(a, seq, (item - seq * a.num_splits) * a.pages_per_split, first_id);
+    w.it = fixed_item(a, item);
+    make_uniform(w.it);
+    w.item_end = 1;
+    w.g_end = 1;
+    return w.it.b >= 0;
+  }
+  bool ids_loaded = false;
+  int g = 0;
+  if (a.spec_pages > 0) {
+    // Every sequence spec_pages pages: sequence b starts at b * spec_pages;
+    // the item size comes from the host. The first piece's ids go out with
+    // the lengths (index clamped: an item past the batch never uses them).
+    const int P = a.spec_pages;
+#pragma unroll
+    for (int k = 0; k < kSeqPerLane; ++k) pb.start[k] = min(64 * k + lane, a.batch) * P;
+    pb.total = a.batch * P;
+    pb.P = v.spec_pps;
+    if (v.writer && threadIdx.x < 64) {
+#pragma unroll
+      for (int k = 0; k < kSeqPerLane; ++k) {
+        const int sq = 64 * k + lane;
+        if (sq < a.batch) {
+          const int i0 = pb.start[k] / pb.P;
+          v.table[sq] = SeqSplits{i0 + sq, (pb.start[k] + P - 1) / pb.P - i0 + 1};
+        }
+      }
+    }
+    // Paired items: the shared boundary of items 2k and 2k + 1 moves by d
+    // pages; delta is the fixed one, or (adaptive pairs) the record's, read
+    // with the lengths, the first ids after.
+    w.paired = kPairs && a.pair_items != 0;
+    int g0 = item * pb.P;
+    w.item_end = g0 + pb.P;
+    if (w.paired) {
+      float dl = kPairDeltaFixed;
+      if (a.pair_items == kPairsAdaptive) {
+        const float2 rec = *(const float2*)a.tune;
+        dl = __float_as_uint(rec.x) == kTuneMagic ? rec.y : 0.f;
+      }
+      load_lengths(a, pb.len);
+      dl = dl == dl ? fminf(fmaxf(dl, -kPairDeltaMax), kPairDeltaMax) : 0.f;
+      // Both items of a pair stay within kMaxSplitPages (the page-id table).
+      const int dmax = kMaxSplitPages - pb.P;
+      const int d = __builtin_amdgcn_readfirstlane(
+          min(max((int)rintf((float)pb.P * dl), -dmax), dmax));
+      g0 = (item >> 1) * 2 * pb.P + ((item & 1) ? pb.P + d : 0);
+      w.item_end = (item >> 1) * 2 * pb.P + ((item & 1) ? 2 * pb.P : pb.P + d);
+    }
+    g0 = __builtin_amdgcn_readfirstlane(g0);
+    const int b0 = min(g0 / P, a.batch - 1);
+    load_first_ids<D>(a, b0, g0 - b0 * P, first_id);
+    if (!w.paired) load_lengths(a, pb.len);
+    bool differs = false;
+#pragma unroll
+    for (int k = 0; k < kSeqPerLane; ++k)
+      differs |= 64 * k + lane < a.batch && pages_of(a, pb.len[k]) != P;
+    if (__any(differs)) {
+      packed_plan(a, v, pb, v.writer);  // rewrites the table
+      w.paired = false;
+    } else {
+      ids_loaded = true;
+    }
+    if (w.paired) g = g0;
+  } else {
+    load_lengths(a, pb.len);
+    packed_plan(a, v, pb, v.writer);
+  }
+  if (!w.paired) {
+    g = item * pb.P;
+    w.item_end = g + pb.P;
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  w.g_end = __builtin_amdgcn_readfirstlane(min(w.item_end, pb.total));
+  if (!piece_at(a, w, item, g)) return false;  // uniform
+  if (!ids_loaded) load_first_ids<D>(a, w.it.b, w.it.p_begin, first_id);
+  return true;
+}
+
+// Runs `piece(range, first_id)` for every piece of workgroup item `item`.
+// Consecutive pieces are separated by a barrier (they reuse the workgroup's LDS).
+// Returns whether the item ran as a paired item (every workgroup of a call
+// returns the same).
 template <int D, typename Piece>
 __device__ __forceinline__ bool for_each_piece(const PartialArgs& a, const PlanView& v, int item,
                                                Piece&& piece) {
-  const int lane = threadIdx.x & 63;
   const bool balanced = is_balanced(a.pages_per_split);
   int first_id[D];
-  auto load_first_ids = [&](int seq, int p0) {
-    const int32_t* row = a.block_tables + (size_t)max(seq, 0) * a.bt_stride;
-#pragma unroll
-    for (int j = 0; j < D; ++j)
-      first_id[j] = row[min(max(p0 + j, 0), a.max_pages - 1) >> a.page_shift];
-  };
-  PackedBatch pb;
-  ItemRange it;
-  bool ids_loaded = false;
-  int g = 0, g_end = 1;  // global pages still to visit (fixed plan: one piece)
-  int item_end = 0;      // balanced plan: where the item ends
-  bool paired = false;
-  if (!balanced) {
-    const int seq = item / a.num_splits;
-    load_first_ids(seq, (item - seq * a.num_splits) * a.pages_per_split);
-    ids_loaded = true;
-    it = fixed_item(a, item);
-  } else {
-    if (a.spec_pages > 0) {
-      // Every sequence spec_pages pages: sequence b starts at b * spec_pages;
-      // the item size comes from the host. The first piece's ids go out with
-      // the lengths (index clamped: an item past the batch never uses them).
-      const int P = a.spec_pages;
-#pragma unroll
-      for (int k = 0; k < kSeqPerLane; ++k) pb.start[k] = min(64 * k + lane, a.batch) * P;
-      pb.total = a.batch * P;
-      pb.P = v.spec_pps;
-      if (v.writer && threadIdx.x < 64) {
-#pragma unroll
-        for (int k = 0; k < kSeqPerLane; ++k) {
-          const int sq = 64 * k + lane;
-          if (sq < a.batch) {
-            const int i0 = pb.start[k] / pb.P;
-            v.table[sq] = SeqSplits{i0 + sq, (pb.start[k] + P - 1) / pb.P - i0 + 1};
-          }
-        }
-      }
-      // Paired items: the shared boundary of items 2k and 2k + 1 moves by d
-      // pages; delta is the fixed one, or (adaptive pairs) the record's, read
-      // with the lengths, the first ids after.
-      paired = a.pair_items != 0;
-      int g0 = item * pb.P;
-      item_end = g0 + pb.P;
-      if (paired) {
-        float dl = kPairDeltaFixed;
-        if (a.pair_items == kPairsAdaptive) {
-          const float2 rec = *(const float2*)a.tune;
-          dl = __float_as_uint(rec.x) == kTuneMagic ? rec.y : 0.f;
-        }
-        load_lengths(a, pb.len);
-        dl = dl == dl ? fminf(fmaxf(dl, -kPairDeltaMax), kPairDeltaMax) : 0.f;
-        // Both items of a pair stay within kMaxSplitPages (the page-id table).
-        const int dmax = kMaxSplitPages - pb.P;
-        const int d = __builtin_amdgcn_readfirstlane(
-            min(max((int)rintf((float)pb.P * dl), -dmax), dmax));
-        g0 = (item >> 1) * 2 * pb.P + ((item & 1) ? pb.P + d : 0);
-        item_end = (item >> 1) * 2 * pb.P + ((item & 1) ? 2 * pb.P : pb.P + d);
-      }
-      const int b0 = min(g0 / P, a.batch - 1);
-      load_first_ids(b0, g0 - b0 * P);
-      if (!paired) load_lengths(a, pb.len);
-      bool differs = false;
-#pragma unroll
-      for (int k = 0; k < kSeqPerLane; ++k)
-        differs |= 64 * k + lane < a.batch && pages_of(a, pb.len[k]) != P;
-      if (__any(differs)) {
-        packed_plan(a, v, pb, v.writer);  // rewrites the table
-        paired = false;
-      } else {
-        ids_loaded = true;
-      }
-      if (paired) g = g0;
-    } else {
-      load_lengths(a, pb.len);
-      packed_plan(a, v, pb, v.writer);
+  ItemWalk w;
+  bool more = first_piece<D, true>(a, v, item, w, first_id);
+  while (more) {  // uniform
+    piece(w.it, first_id);
+    more = balanced && piece_at(a, w, item, w.it.g_end);
+    if (more) {
+      load_first_ids<D>(a, w.it.b, w.it.p_begin, first_id);
+      __syncthreads();  // the previous piece is done with the LDS
     }
-    if (!paired) {
-      g = item * pb.P;
-      item_end = g + pb.P;
-    }
-    g_end = min(item_end, pb.total);
   }
-  // The same in every lane (readfirstlane tells the compiler, which otherwise
-  // runs the loop under an exec mask).
-  g = __builtin_amdgcn_readfirstlane(g);
-  g_end = __builtin_amdgcn_readfirstlane(g_end);
-  for (bool first = true; g < g_end; first = false) {  // uniform
-    if (balanced) it = packed_piece(a, pb, item, g, item_end);
-    it.paired = paired;
-    it.b = __builtin_amdgcn_readfirstlane(it.b);
-    it.split = __builtin_amdgcn_readfirstlane(it.split);
-    it.p_begin = __builtin_amdgcn_readfirstlane(it.p_begin);
-    it.p_end = __builtin_amdgcn_readfirstlane(it.p_end);
-    it.len = __builtin_amdgcn_readfirstlane(it.len);
-    it.n_valid = __builtin_amdgcn_readfirstlane(it.n_valid);
-    it.slot0 = __builtin_amdgcn_readfirstlane(it.slot0);
-    // A piece has a sequence and at least one page unless the item ends in the
-    // gap before a sequence start (no further pieces then); the check also keeps
-    // the loop finite whatever the inputs.
-    if (balanced && (it.b < 0 || it.p_end <= it.p_begin)) break;
-    // Uniform addresses (the fields above) make the ids uniform values: the
-    // buffer resources built from them stay in scalar registers.
-    if (!ids_loaded) load_first_ids(it.b, it.p_begin);
-    ids_loaded = false;
-    if (!first) __syncthreads();  // the previous piece is done with the LDS
-    piece(it, first_id);
-    g = __builtin_amdgcn_readfirstlane(balanced ? it.g_end : g + 1);
-  }
-  return paired;
+  return w.paired;
 }
 
 // Draft bits of a row of sequence b, draft row qi: bit j = the row sees draft
@@ -1223,6 +1270,73 @@ __device__ __forceinline__ void write_empty_split(const PartialArgs& a, const Ma
   }
 }
 
+// s_waitcnt vmcnt(n) that no memory access is moved across.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_fence() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N < 63 ? N : 63) : "memory");
+}
+
+// One load per lane straight into LDS (gfx950 global_load_lds_*): lane l's 16 (or
+// 4) bytes land at LDS byte address lds + 16 l (4 l). Inline asm for the reason
+// given at load_to_lds: the compiler's wait-count pass must not drain the page
+// ring for it. The callers wait themselves (wait_vmcnt_fence).
+__device__ __forceinline__ void copy16_to_lds(const void* src, unsigned lds) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %[saved], m0\n\t"
+      "s_mov_b32 m0, %[lds]\n\t"
+      "global_load_lds_dwordx4 %[src], off\n\t"
+      "s_mov_b32 m0, %[saved]"
+      : [saved] "=&s"(saved)
+      : [lds] "s"(lds), [src] "v"(src)
+      : "memory");
+}
+__device__ __forceinline__ void copy4_to_lds(const void* src, unsigned lds) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %[saved], m0\n\t"
+      "s_mov_b32 m0, %[lds]\n\t"
+      "global_load_lds_dword %[src], off\n\t"
+      "s_mov_b32 m0, %[saved]"
+      : [saved] "=&s"(saved)
+      : [lds] "s"(lds), [src] "v"(src)
+      : "memory");
+}
+
+// Draft bits held in registers (loaded with draft_bits()).
+template <int NB>
+struct RegBits {
+  unsigned long long b[NB];
+  __device__ __forceinline__ void get(unsigned long long (&dbits)[NB]) const {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) dbits[nb] = b[nb];
+  }
+};
+
+// Draft bits of a wave's rows: the caller's mask words, copied to LDS with the
+// piece's Q (block nb's row r: word w at 32 nb + 16 w + r), or the causal chain.
+// Padding rows get some row's bits; they are never stored.
+template <int NB, int HPW>
+struct StagedBits {
+  const unsigned* words;
+  bool masked;            // the caller's words; else the causal chain
+  bool two;               // two words per row
+  int group, l16;
+  WaveRows<NB, HPW> map;
+  __device__ __forceinline__ void get(unsigned long long (&dbits)[NB]) const {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (masked) {  // uniform
+        dbits[nb] = words[32 * nb + l16];
+        if (two) dbits[nb] |= (unsigned long long)words[32 * nb + 16 + l16] << 32;
+      } else {
+        const int qi = map.row(nb, l16) / group;
+        dbits[nb] = qi >= 63 ? ~0ull : (2ull << qi) - 1ull;
+      }
+    }
+  }
+};
+
 // One workgroup = one (sequence b, split) x WW waves; wave w serves the HPW kv
 // heads from (head_group * WW + w) * HPW with all of their rows (NB blocks of
 // 16; with HPW = 2 either one block, rows 0-7 of the first head and 8-15 of
@@ -1234,11 +1348,27 @@ __device__ __forceinline__ void write_empty_split(const PartialArgs& a, const Ma
 // softmax state and writes its own partials (or, with a single split, the
 // output). Every K/V byte is read by one wave only, so the loads are
 // non-temporal.
+// The page ring runs through the pieces of an item: the next piece's first pages
+// are requested in this one's last turn and its Q and mask words as soon as this
+// one begins, so a sequence end costs the epilogue (about 1 us) and not a drained
+// ring, a second barrier and three round trips (8.7 us at 16 ragged sequences of
+// 2K-32K tokens). Whole calls, before -> after: 64 sequences of up to 512 keys at
+// q_len 2 32.2 -> 27.5 us, 128 of up to 330 40.8 -> 34.3; 32 of up to 1K at q_len 8
+// 36.4 -> 33.5; head dim 64, 4 of 2K, 18.7 -> 16.7 (there each thread also loaded
+// nine page ids for every piece, now one for the item). Long uniform batches, whose
+// items end with their sequences, are unchanged. What bounds it: HBM, and for few
+// pages per item the start-up.
 template <int NB, int D, int WW, int WPE, int HD, typename E, typename KV, int HPW,
           bool RB = false>
 __global__ __launch_bounds__(WW * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void sqa_partial_kernel(PartialArgs a) {
   constexpr int KK = Dims<HD>::KK, MB = Dims<HD>::MB;
+  // The arguments on the way to the first page ids, asked for together (one round
+  // trip): left to itself the compiler loads them where they are first used, six
+  // dependent trips through the scalar cache.
+  asm volatile("" ::"s"(a.block_tables), "s"(a.seq_lens), "s"(a.batch), "s"(a.hkv),
+               "s"(a.num_splits), "s"(a.pages_per_split), "s"(a.bt_stride), "s"(a.max_pages),
+               "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.hg_items[0]));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // blockIdx.x = item * head_groups + head_group, or with items per head group
@@ -1261,77 +1391,110 @@ void sqa_partial_kernel(PartialArgs a) {
 
   const bool balanced = is_balanced(a.pages_per_split);
   const bool single = !balanced && a.num_splits == 1;  // no merge kernel follows
-  static_assert(2 * D + 1 <= kIdPad, "page-id table padding must cover the ring's look-ahead");
-  constexpr int kIdSlots = (kMaxSplitPages + kIdPad + WW * 64 - 1) / (WW * 64);
-  // LDS: the Q fragments of this wave's rows, [wave][nb][kk][lane] (the
-  // B-operand layout; each lane stores exactly the fragments it reads back),
-  // and the piece's page ids: ids of [p_begin, p_end) clamped into the pool,
-  // then -1 for the ring's look-ahead. Waves read ids back a step ahead of
-  // use, so no page waits on a block-table load from memory. sm_stage holds
-  // each wave's results on their way out (the epilogue below).
-  __shared__ u4 sm_q[WW * NB * KK * 64];
-  __shared__ float sm_stage[WW * 16 * (HD + 4)];
-  __shared__ int sm_ids[kIdSlots * WW * 64];
 
-  // Each piece of the work item (one, except where a balanced item spans the
-  // end of a sequence): its page range of one sequence, with the ids of its
-  // first D pages already requested.
-  for_each_piece<D>(a, view, item, [&](const ItemRange& it, const int (&first_id)[D]) {
+  // The page loop of each of the three forms below (see there).
+  constexpr bool kPipelined = NB >= 2 && D >= 3 && NB * HD <= 256;
+  constexpr bool kPairSteps = __is_same(E, ElemF16) && KV::kBytes == 1 && HD == 128 &&
+                              NB == 4 && HPW == 1 && D % 2 == 0;
+  constexpr bool kRingBatch = RB && KV::kBytes == 2 && HD <= 128;
+  constexpr bool kQRegs =
+      ((NB == 4 && KV::kBytes == 1) || HD == 256) && HPW == 1 && !kPipelined;
+
+  // LDS, all of it a wave's own but the page ids: the Q fragments of the wave's
+  // rows, [buffer][nb][kk][lane] (the B-operand layout), and their draft-mask
+  // words, twice (the piece at hand and the next one; once where the loop holds
+  // Q in registers); the item's page ids (below); the results on their way out.
+  constexpr int kQBufs = kQRegs || kPairSteps ? 1 : 2;
+  constexpr int kQLds = NB * KK * 64;                    // u4 per wave and buffer
+  constexpr int kBitsLds = NB * 32 < 64 ? 64 : NB * 32;  // dwords per wave and buffer
+  // Ids of the item's pages in walking order, each piece padded with -1 to whole
+  // turns of the ring: at most kMaxSplitPages pages in kMaxBalancedBatch pieces.
+  constexpr int kIds = kMaxSplitPages + kMaxBalancedBatch * (D - 1) + 2 * D + 2;
+  __shared__ u4 sm_q[WW * kQBufs * kQLds];
+  __shared__ unsigned sm_bits[WW * 2 * kBitsLds];
+  __shared__ float sm_stage[WW * 16 * (HD + 4)];
+  __shared__ int sm_ids[kIds];
+
+  // The first piece of the item and the ids of its first D pages, requested.
+  ItemWalk walk;
+  int first_id[D];
+  if (!first_piece<D, false>(a, view, item, walk, first_id)) return;  // uniform
+  ItemRange it = walk.it;
+  const size_t first_slot = (size_t)it.slot0 + it.split;
+  if (it.p_begin >= it.p_end && !single) {  // fixed plan only
+    if (active) write_empty_split<NB>(a, map, first_slot, it.n_valid == 1 ? -1.f : 0.f);
+    return;  // uniform
+  }
   const int tid = piece_tid();
   const int lane = tid & 63;
   const int g16 = lane >> 4;
   const int l16 = lane & 15;
-  const int b = max(it.b, 0);
-  const int split = it.split;
-  const int len = it.len;
-  const int p_begin = it.p_begin;
-  const int p_end = it.p_end;
-  const int32_t* bt_row = a.block_tables + (size_t)b * a.bt_stride;
   const int shift = a.page_shift;
   const int sub_mask = (1 << shift) - 1;
-  if (it.b < 0) return;  // uniform: no work item
-  // A sequence with at most one split is finished here; otherwise this
-  // workgroup leaves a partial for the merge kernel.
-  const bool direct = it.n_valid <= 1;
-  const size_t slot = (size_t)it.slot0 + split;
-  if (p_begin >= p_end && !single) {  // fixed plan only
-    if (active) write_empty_split<NB>(a, map, slot, it.n_valid == 1 ? -1.f : 0.f);
-    return;  // uniform
-  }
-  const int n_split = p_end - p_begin;
-  const int n_pages = active ? n_split : 0;
+  auto padded = [](int n) { return (n + D - 1) / D * D; };
 
-  // Second: Q fragments, the rest of the split's page ids and the first D
-  // pages, all in flight at once (Q and ids first, so waiting for them leaves
-  // the page loads outstanding).
-  u4 qreg[NB][KK];
-  unsigned long long dbits[NB];
+  // Q fragments and mask words of a piece's rows on their way into buffer `buf`
+  // (padding rows take some row's, unused).
+  u4* my_q = sm_q + wave * kQBufs * kQLds;
+  unsigned* my_bits = sm_bits + wave * 2 * kBitsLds;
+  auto fetch_rows = [&](int b, int buf) {
+    if (!active) return;  // uniform
+    const int t = piece_tid() & 63;
+    const int tg = t >> 4, tl = t & 15;
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    // Loads are unconditional from an in-bounds address (padding rows and idle
-    // waves read row 0 of kv head 0) and the value is selected afterwards, so
-    // no lane-divergent branch splits the load stream.
-    const int r = map.row(nb, l16);
-    const bool real = map.real(nb, l16);
-    const int qi = real ? r / a.group : 0;
-    const int gg = real ? r - qi * a.group : 0;
-    const int hh = real ? map.head(nb, l16) * a.group + gg : 0;
-    const _Float16* qp = a.q + ((size_t)(b * a.q_len + qi) * a.hq + hh) * HD;
+    for (int nb = 0; nb < NB; ++nb) {
+      const int r = map.row(nb, tl);
+      const bool real = map.real(nb, tl);
+      const int qi = real ? r / a.group : 0;
+      const int gg = real ? r - qi * a.group : 0;
+      const int hh = (real ? map.head(nb, tl) : map.kvh) * a.group + gg;
+      const _Float16* qp = a.q + ((size_t)(b * a.q_len + qi) * a.hq + hh) * HD;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      const u4 x = *(const u4*)(qp + KV::q_dims(kk, g16));
-      qreg[nb][kk] = real ? x : u4{0u, 0u, 0u, 0u};
+      for (int kk = 0; kk < KK; ++kk)
+        copy16_to_lds(qp + KV::q_dims(kk, tg),
+                      (unsigned)(size_t)(my_q + ((buf % kQBufs) * NB + nb) * KK * 64 + kk * 64));
     }
-    dbits[nb] = draft_bits(a, b, qi, real);
-  }
-  int idreg[kIdSlots];
-  const int last_id = n_split > 0 ? n_split - 1 : 0;  // p_begin + last_id < max_pages
+    if (a.draft_mask != nullptr) {  // uniform
 #pragma unroll
-  for (int k = 0; k < kIdSlots; ++k) {
-    const int i = tid + k * WW * 64;
-    const int x = bt_row[(p_begin + min(i, last_id)) >> shift];
-    idreg[k] = i < n_split ? x : -1;
+      for (int i = 0; i < kBitsLds / 64; ++i) {
+        // Lane t fills dword 64 i + t: block nb, word w, row slot r.
+        const int nb = min(2 * i + (t >> 5), NB - 1), w = (t >> 4) & 1;
+        const int qi = map.real(nb, tl) ? map.row(nb, tl) / a.group : 0;
+        copy4_to_lds(a.draft_mask + (size_t)(b * a.q_len + qi) * a.mask_words +
+                         (a.mask_words > 1 ? w : 0),
+                     (unsigned)(size_t)(my_bits + buf * kBitsLds + 64 * i));
+      }
+    }
+  };
+
+  // Ids of the item's pages, entry tid of each run of WW * 64: the address in the
+  // block table, found piece by piece, or -1 (padding). Long items (more than one
+  // run, so hundreds of pages) fill all but the first run here; the first run's
+  // loads go out with Q and the first pages below.
+  const int32_t* ids_base =
+      balanced ? a.block_tables : a.block_tables + (size_t)it.b * a.bt_stride;
+  int n_flat = 0;
+  auto id_at = [&](int e) {
+    walk.it = it;
+    int at = -1;
+    n_flat = 0;
+    do {  // uniform
+      const int n = walk.it.p_end - walk.it.p_begin;
+      const int rel = e - n_flat;
+      if (rel >= 0 && rel < n)
+        at = (balanced ? walk.it.b * a.bt_stride : 0) + ((walk.it.p_begin + rel) >> shift);
+      n_flat += padded(n);
+    } while (balanced && piece_at(a, walk, item, walk.it.g_end));
+    return at;
+  };
+  const int at0 = id_at(tid);
+  for (int e = WW * 64; e < n_flat; e += WW * 64) {  // uniform
+    const int at = id_at(e + tid);
+    const int x = ids_base[max(at, 0)];
+    if (e + tid < kIds) sm_ids[e + tid] = at >= 0 ? clamp_page(x, a.num_pages) : -1;
   }
+  const int id0 = ids_base[max(at0, 0)];
+  fetch_rows(it.b, 0);
 
   // K/V pages are read with buffer loads: the resource (4 SGPRs) is rebuilt per
   // page at the page's base address and bounded to the page, and the lane
@@ -1363,25 +1526,48 @@ void sqa_partial_kernel(PartialArgs a) {
     if constexpr (HPW == 2) KV::load(pg[HPW - 1], kr, vr, k_lane + head1, v_lane + head1, tok_bytes);
   };
   // Ring of D pages in flight: page i is processed from slot i % D, which is
-  // then refilled with page i + D.
+  // then refilled with page i + D, past a piece's (padded) end with the next
+  // piece's first pages: the ring runs through the piece boundaries of an item.
   typename KV::Regs ring[D][HPW];
 #pragma unroll
   for (int j = 0; j < D; ++j) {
-    load_page(j < n_pages ? clamp_page(first_id[j], a.num_pages) : -1, p_begin + j, ring[j]);
+    load_page(active && j < it.p_end - it.p_begin ? clamp_page(first_id[j], a.num_pages) : -1,
+              it.p_begin + j, ring[j]);
   }
+  sm_ids[tid] = at0 >= 0 ? clamp_page(id0, a.num_pages) : -1;
+  __syncthreads();  // the ids are in LDS: the item's only barrier
+  if (!active) return;  // uniform over the wave: no barrier follows
+  auto page_id = [&](int i) -> int {
+    const int x = sm_ids[i];
+    return i < n_flat ? x : -1;
+  };
+  const bool upper = l16 >= 8;
+  static_assert(WW * 64 <= kIds, "the first run of ids fits the table");
 
-  u4* my_q = sm_q + wave * NB * KK * 64;
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) my_q[(nb * KK + kk) * 64 + lane] = qreg[nb][kk];
-  }
-#pragma unroll
-  for (int k = 0; k < kIdSlots; ++k) {
-    const int i = tid + k * WW * 64;
-    sm_ids[i] = idreg[k] >= 0 ? clamp_page(idreg[k], a.num_pages) : -1;
-  }
-  auto page_id = [&](int i) -> int { return active ? sm_ids[i] : -1; };
+  // Each piece of the work item (one, except where a balanced item spans the end
+  // of a sequence): its page range of one sequence, ids from table entry f on.
+  int f = 0;
+  for (int buf = 0;; buf ^= 1) {
+  const int len = it.len;
+  const int p_begin = it.p_begin;
+  const int n_pages = it.p_end - it.p_begin;
+  const int n_padded = padded(max(n_pages, 0));
+  // A sequence with at most one split is finished here; otherwise this
+  // workgroup leaves a partial for the merge kernel.
+  const bool direct = it.n_valid <= 1;
+  const size_t slot = (size_t)it.slot0 + it.split;
+  // The piece after this one: its first pages enter the ring during this one's
+  // last turn, its Q fragments now (with one buffer: once this piece's are in
+  // registers).
+  walk.it = it;
+  const bool more = balanced && piece_at(a, walk, item, it.g_end);
+  const int next_begin = walk.it.p_begin;
+  if (kQBufs == 2 && more) fetch_rows(walk.it.b, buf ^ 1);
+  // This piece's Q and mask words are in LDS: D pages were requested after them.
+  wait_vmcnt_fence<D * HPW * KV::kLoads>();
+  const u4* q_lds = my_q + (buf % kQBufs) * kQLds;
+  const StagedBits<NB, HPW> bits{my_bits + buf * kBitsLds, a.draft_mask != nullptr,
+                                 a.mask_words > 1, a.group, l16, map};
   // Pages holding a token >= mask_from (draft block or past the end) are masked.
   const int mask_from = len - a.q_len;
 
@@ -1395,8 +1581,17 @@ void sqa_partial_kernel(PartialArgs a) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) st.acc[mb][nb] = f4{0.f, 0.f, 0.f, 0.f};
   }
-
-  __syncthreads();  // sm_q and sm_ids written
+  u4 qf[kQRegs || kPairSteps ? NB : 1][KK];
+  if constexpr (kQRegs || kPairSteps) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) qf[nb][kk] = q_lds[(nb * KK + kk) * 64 + lane];
+    if (more) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      fetch_rows(walk.it.b, buf ^ 1);
+    }
+  }
 
   // With two or four row blocks whose accumulators take at most 64 VGPRs
   // (NB * HD <= 256) the page loop is software-pipelined: the scores of page
@@ -1409,18 +1604,13 @@ void sqa_partial_kernel(PartialArgs a) {
   // us), with a ring of 2 the wait is longer (head dim 256: 662 -> 916 us),
   // and at one block there is little softmax to hide (e4m3 head dim 64 q4:
   // -1.5%).
-  constexpr bool kPipelined = NB >= 2 && D >= 3 && NB * HD <= 256;
   // fp16 queries over an e4m3 cache at 64 rows and head dim 128 take the
   // pages two at a time (pair_finish).
-  constexpr bool kPairSteps = __is_same(E, ElemF16) && KV::kBytes == 1 && HD == 128 &&
-                              NB == 4 && HPW == 1 && D % 2 == 0;
   // A piece that fits the ring in one softmax step (below), in the RB
   // instantiations only (the host picks them for plans whose pieces fit the
   // ring: with the step in it, the kernel's page loop for long pieces ran 1-2%
   // slower): 16-bit K/V, whose ring registers the MFMAs read as they are.
-  constexpr bool kRingBatch = RB && KV::kBytes == 2 && HD <= 128;
-  const bool upper = l16 >= 8;
-  int next_pid = page_id(D);
+  int next_pid = page_id(f + D);
   if constexpr (kPairSteps) {
     // The Q fragments stay in registers for the whole loop (16 x 4 dwords; the
     // ring, scores and accumulators take the 256 arch VGPRs, so they live in
@@ -1429,12 +1619,8 @@ void sqa_partial_kernel(PartialArgs a) {
     // v_accvgpr_mov per 4 pages); the empty asm below states that the values
     // sit in AGPRs at that point, and the copies are gone (cfg3 shape q16:
     // 217.8 -> 209.6 us).
-    u4 qf[NB][KK];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) qf[nb][kk] = my_q[(nb * KK + kk) * 64 + lane];
     for (int i = 0; i < n_pages; i += D) {
+      const int p_ahead = i + D < n_padded ? p_begin + i + D : next_begin;
 #pragma unroll
       for (int j = 0; j < D; j += 2) {
         const int ii = i + j;
@@ -1468,14 +1654,14 @@ void sqa_partial_kernel(PartialArgs a) {
               for (int kk = 0; kk < KK; ++kk) s1[nb] = E::mma_qk(k1.k[0][kk], qf[nb][kk], s1[nb]);
             }
           }
-          pair_finish<NB>(st, s0, s1, ring[j][0], ring[j + 1][0], ii + 1 < n_pages, dbits,
+          pair_finish<NB>(st, s0, s1, ring[j][0], ring[j + 1][0], ii + 1 < n_pages, bits,
                           mask_from, p * kPageSize + 4 * g16, len, masked, a.scale_log2);
         }
         const int pid0 = next_pid;
-        const int pid1 = page_id(ii + D + 1);
-        next_pid = page_id(ii + D + 2);
-        load_page(pid0, p_begin + ii + D, ring[j]);
-        load_page(pid1, p_begin + ii + D + 1, ring[j + 1]);
+        const int pid1 = page_id(f + ii + D + 1);
+        next_pid = page_id(f + ii + D + 2);
+        load_page(pid0, p_ahead + j, ring[j]);
+        load_page(pid1, p_ahead + j + 1, ring[j + 1]);
       }
     }
   } else if (kRingBatch && n_pages <= D) {  // uniform: the whole piece is in the ring
@@ -1490,7 +1676,7 @@ void sqa_partial_kernel(PartialArgs a) {
     PageV<HD, HPW> pvb[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      page_scores<NB, HD, E, KV, HPW>(sb[j], widen_k<E, KV, HD, HPW>(ring[j]), my_q, lane, upper);
+      page_scores<NB, HD, E, KV, HPW>(sb[j], widen_k<E, KV, HD, HPW>(ring[j]), q_lds, lane, upper);
       pvb[j] = widen_v<E, KV, HD, HPW>(ring[j]);
     }
     float lm[NB];
@@ -1503,6 +1689,8 @@ void sqa_partial_kernel(PartialArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) sb[j][nb] = f4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
       } else if ((p + 1) * kPageSize > mask_from) {  // uniform
+        unsigned long long dbits[NB];
+        bits.get(dbits);
         mask_page<NB, HD, HPW>(sb[j], pvb[j], dbits, mask_from, p * kPageSize + 4 * g16, len);
       }
 #pragma unroll
@@ -1512,25 +1700,21 @@ void sqa_partial_kernel(PartialArgs a) {
 #pragma unroll
     for (int j = 0; j < D; ++j)
       if (j < n_pages) page_pv<NB, HD, E, KV, HPW>(st, sb[j], pvb[j], upper, a.scale_log2);
+    if (more) {  // uniform
+#pragma unroll
+      for (int j = 0; j < D; ++j) load_page(page_id(f + D + j), next_begin + j, ring[j]);
+    }
   } else {
   f4 s_cur[NB];
   if constexpr (kPipelined)
-    page_scores<NB, HD, E, KV, HPW>(s_cur, widen_k<E, KV, HD, HPW>(ring[0]), my_q, lane, upper);
+    page_scores<NB, HD, E, KV, HPW>(s_cur, widen_k<E, KV, HD, HPW>(ring[0]), q_lds, lane, upper);
   // 64 rows over e4m3 outside the page pairs (bf16 queries), and head dim 256:
   // the Q fragments held in AGPRs for the loop, pinned there as in the pair
   // loop (the compiler had copied them between AGPR sets every page; cfg3
   // shape: bf16 / e4m3 q16 283.7 -> 271.0 us, head dim 256 q8 680.5 -> 668.7
   // us, e4m3 324.2 -> 322.2 us).
-  constexpr bool kQRegs =
-      ((NB == 4 && KV::kBytes == 1) || HD == 256) && HPW == 1 && !kPipelined;
-  u4 qf[kQRegs ? NB : 1][KK];
-  if constexpr (kQRegs) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) qf[nb][kk] = my_q[(nb * KK + kk) * 64 + lane];
-  }
   for (int i = 0; i < n_pages; i += D) {
+    const int p_ahead = i + D < n_padded ? p_begin + i + D : next_begin;
 #pragma unroll
     for (int j = 0; j < D; ++j) {
       const int ii = i + j;
@@ -1541,9 +1725,9 @@ void sqa_partial_kernel(PartialArgs a) {
           // Slot (j + 1) % D holds page ii + 1 (a zero page past the split).
           f4 s_next[NB];
           page_scores<NB, HD, E, KV, HPW>(s_next, widen_k<E, KV, HD, HPW>(ring[(j + 1) % D]),
-                                          my_q, lane, upper);
+                                          q_lds, lane, upper);
           PageV<HD, HPW> pv = widen_v<E, KV, HD, HPW>(ring[j]);
-          page_finish<NB, HD, E, KV, HPW>(st, s_cur, pv, upper, dbits, mask_from,
+          page_finish<NB, HD, E, KV, HPW>(st, s_cur, pv, upper, bits, mask_from,
                                           p * kPageSize + 4 * g16, len, masked, a.scale_log2);
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) s_cur[nb] = s_next[nb];
@@ -1563,22 +1747,24 @@ void sqa_partial_kernel(PartialArgs a) {
                 s_cur[nb] = E::mma_qk(kf.k[0][kk], qf[nb][kk], s_cur[nb]);
             }
           } else {
-            page_scores<NB, HD, E, KV, HPW>(s_cur, kf, my_q, lane, upper);
+            page_scores<NB, HD, E, KV, HPW>(s_cur, kf, q_lds, lane, upper);
           }
-          page_finish<NB, HD, E, KV, HPW>(st, s_cur, pv, upper, dbits, mask_from,
+          page_finish<NB, HD, E, KV, HPW>(st, s_cur, pv, upper, bits, mask_from,
                                           p * kPageSize + 4 * g16, len, masked, a.scale_log2);
         }
       }
       const int pid = next_pid;
-      next_pid = page_id(ii + D + 1);
-      load_page(pid, p_begin + ii + D, ring[j]);
+      next_pid = page_id(f + ii + D + 1);
+      load_page(pid, p_ahead + j, ring[j]);
     }
   }
   }
-  if (active)
-    write_results<NB, HD, E>(a, st, sm_stage + wave * 16 * (HD + 4), map, direct,
-                             !single && !balanced, b, slot + slot_base, slot_heads, head0);
-  });
+  write_results<NB, HD, E>(a, st, sm_stage + wave * 16 * (HD + 4), map, direct,
+                           !single && !balanced, it.b, slot + slot_base, slot_heads, head0);
+  if (!more) break;  // uniform
+  f += n_padded;
+  it = walk.it;
+  }
 }
 
 // The rows of one wave of the 8-wave kernel: rows base .. base + 31 of kv head
@@ -1747,7 +1933,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
 
   // Q fragments (kept in registers), draft bits, then the split's page ids.
   u4 qreg[NB][KK];
-  unsigned long long dbits[NB];
+  RegBits<NB> bits;
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     const int r = map.row(nb, l16);
@@ -1761,7 +1947,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
       const u4 x = *(const u4*)(qp + KV::q_dims(kk, g16));
       qreg[nb][kk] = real ? x : u4{0u, 0u, 0u, 0u};
     }
-    dbits[nb] = draft_bits(a, b, qi, real);
+    bits.b[nb] = draft_bits(a, b, qi, real);
   }
   int idreg[kIdSlots];
   const int last_id = n_split > 0 ? n_split - 1 : 0;
@@ -1837,7 +2023,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) sc[nb] = E::mma_qk(kf.k[0][kk], qreg[nb][kk], sc[nb]);
           }
-          page_finish<NB, HD, E, KV, 1>(st, sc, pv, false, dbits, mask_from,
+          page_finish<NB, HD, E, KV, 1>(st, sc, pv, false, bits, mask_from,
                                         p * kPageSize + 4 * g16, len, masked, a.scale_log2);
         }
       }
