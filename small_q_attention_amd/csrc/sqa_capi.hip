@@ -452,6 +452,11 @@ int run_attention(const sqa_attention_args& a) {
   pa.out_scale = a.out_scale;
   pa.bf16 = a.dtype == SQA_DTYPE_BF16;
   pa.kv_fp8 = kv_fp8;
+  const sqa::LaunchShape shape = sqa::launch_shape((int)rows, num_kv_heads, head_dim);
+  pa.by_head_groups = sqa::fast_div((num_kv_heads + shape.heads - 1) / shape.heads);
+  pa.by_splits = sqa::fast_div(num_splits);
+  pa.by_spec_pages = sqa::fast_div(spec_pages > 0 ? spec_pages : 1);
+  pa.by_group = sqa::fast_div(group);
 
   hipError_t e;
   if (ev && (e = hipEventRecord(ev[0], s)) != hipSuccess) return hip_fail(e, "hipEventRecord");
@@ -479,6 +484,11 @@ int run_attention(const sqa_attention_args& a) {
     ma.hg_items[0] = pa.hg_items[0];
     ma.hg_items[1] = pa.hg_items[1];
     ma.hg_spec_pps1 = pa.hg_spec_pps1;
+    ma.by_hq = sqa::fast_div(num_query_heads);
+    ma.by_seq_rows = sqa::fast_div(q_len * num_query_heads);
+    ma.by_group = pa.by_group;
+    ma.by_spec_pps = sqa::fast_div(ma.spec_pps > 0 ? ma.spec_pps : 1);
+    ma.by_spec_pps1 = sqa::fast_div(ma.hg_spec_pps1 > 0 ? ma.hg_spec_pps1 : 1);
     ma.out_scale = a.out_scale;
     ma.bf16 = pa.bf16;
     ma.tune = pa.pair_items == sqa::kPairsAdaptive ? pa.tune : nullptr;

@@ -28,6 +28,23 @@ struct SeqSplits {
   int count;
 };
 
+// Division by a value the host knows, for 0 <= n < 2^31: n * mul >> shift with mul =
+// floor(2^shift / d) + 1, shift = 31 + ceil(log2 d) (mul exceeds 2^shift / d by at
+// most 1, so the quotient by less than 2^31 / 2^shift <= 1 / d: exact). A division
+// by a run-time value is some 20 dependent instructions, about 0.1 us for a lone
+// wave, and a call's way to its first load had five.
+struct FastDiv {
+  unsigned mul, shift;
+};
+inline FastDiv fast_div(unsigned d) {
+  unsigned l = 0;
+  while ((1ull << l) < d) ++l;
+  return {(unsigned)((1ull << (31 + l)) / d + 1), 31 + l};
+}
+__host__ __device__ inline int operator/(int n, FastDiv d) {
+  return (int)(((unsigned long long)(unsigned)n * d.mul) >> d.shift);
+}
+
 // Everything the split-KV partial kernel needs. Element counts, not bytes.
 //
 // Two split plans. Fixed (pages_per_split > 0): sequence b owns slots
@@ -161,6 +178,10 @@ struct PartialArgs {
   int hg_spec_pps1;           // with hg_items: head group 1's item size (spec_pps: group 0's)
   float* tune;                // adaptive paired items: {magic, delta, stamp, -} then per
                               // workgroup {loop ticks, pages}
+  FastDiv by_head_groups;     // workgroups per item
+  FastDiv by_splits;          // num_splits
+  FastDiv by_spec_pages;      // spec_pages (where it is > 0)
+  FastDiv by_group;           // group
   float scale_log2;           // softmax scale * log2(e)
   float out_scale;            // multiplier applied to the normalised output
   int bf16;                   // element type of Q and out (and of K, V unless kv_fp8): 0 fp16, 1 bf16
@@ -195,6 +216,8 @@ struct MergeArgs {
   int hg_spec_pps1; // as PartialArgs::hg_spec_pps1
   float out_scale;
   int bf16;
+  FastDiv by_hq, by_seq_rows, by_group;  // hq, q_len * hq (a sequence's rows), group
+  FastDiv by_spec_pps, by_spec_pps1;     // spec_pps, hg_spec_pps1 (where they are > 0)
   float* tune;      // adaptive paired items: the delta record to update (null: none)
   int tune_records; // workgroup records after it
 };

@@ -184,14 +184,39 @@ __device__ __forceinline__ void store_through(void* p, unsigned long long x) {
   __hip_atomic_store((unsigned long long*)p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// x of the lower and the upper of two 16-lane rows (kOff 16: rows 0 and 1, and 2
+// and 3) or of two 32-lane halves (kOff 32), each in all of their lanes: one
+// v_permlane swap of x with itself, no LDS permute.
+struct LanePair {
+  float lo, hi;
+};
+template <int kOff>
+__device__ __forceinline__ LanePair lane_pair(float x) {
+  static_assert(kOff == 16 || kOff == 32, "rows or halves of a wave");
+  const unsigned v = __builtin_bit_cast(unsigned, x);
+  unsigned lo, hi;
+  if constexpr (kOff == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    lo = r[0];
+    hi = r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    lo = r[0];
+    hi = r[1];
+  }
+  return {__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+}
+
 __device__ __forceinline__ float xor_max(float x) {
-  x = fmaxf(x, __shfl_xor(x, 16));
-  return fmaxf(x, __shfl_xor(x, 32));
+  const LanePair a = lane_pair<16>(x);
+  const LanePair b = lane_pair<32>(fmaxf(a.lo, a.hi));
+  return fmaxf(b.lo, b.hi);
 }
 
 __device__ __forceinline__ float xor_sum(float x) {
-  x += __shfl_xor(x, 16);
-  return x + __shfl_xor(x, 32);
+  const LanePair a = lane_pair<16>(x);
+  const LanePair b = lane_pair<32>(a.lo + a.hi);
+  return b.lo + b.hi;
 }
 
 // Buffer-resource word 3 for gfx9-family raw (untyped, 32-bit) accesses.
@@ -691,7 +716,7 @@ struct ItemRange {
   int p_begin;  // first page (logical index within the sequence)
   int p_end;    // one past the last page
   int len;      // seq_lens[b], clamped to >= 0
-  int n_valid;  // splits of this sequence that own pages
+  int n_valid;  // splits of this sequence that own pages: 0, 1 or more (then 2)
   int slot0;    // partial slot of split 0 of this sequence
   int g_end;    // balanced plan: where the piece ends along the item's pages
   int paired;   // a paired item of the expected-page plan (its loop time is timed)
@@ -708,13 +733,13 @@ __device__ __forceinline__ int scalar_load(const int32_t* p) {
 // Fixed plan: sequence b owns slots b * num_splits + s.
 __device__ __forceinline__ ItemRange fixed_item(const PartialArgs& a, int item) {
   ItemRange r;
-  r.b = item / a.num_splits;
+  r.b = item / a.by_splits;
   r.split = item - r.b * a.num_splits;
   r.p_begin = r.split * a.pages_per_split;
   r.len = max(scalar_load(a.seq_lens + r.b), 0);
   const int pages = min((r.len + kPageSize - 1) / kPageSize, a.max_pages);
   r.p_end = min(r.p_begin + a.pages_per_split, pages);
-  r.n_valid = min((pages + a.pages_per_split - 1) / a.pages_per_split, a.num_splits);
+  r.n_valid = min(pages > a.pages_per_split ? 2 : (int)(pages > 0), a.num_splits);
   r.slot0 = r.b * a.num_splits;
   r.g_end = 0;
   r.paired = 0;
@@ -836,9 +861,9 @@ __device__ __forceinline__ void packed_plan(const PartialArgs& a, const PlanView
     int vstart[kSeqPerLane];
 #pragma unroll
     for (int k = 0; k < kSeqPerLane; ++k) {
-      const int gap = pages[k] > 0 && pb.start[k] % pb.P != 0 ? seam : 0;
       vstart[k] = pb.start[k] + gap_base;
       if (k < groups) {
+        const int gap = pages[k] > 0 && pb.start[k] % pb.P != 0 ? seam : 0;
         const int incl = wave_inclusive_scan_int(gap);
         vstart[k] += incl;
         gap_base += __builtin_amdgcn_readlane(incl, 63);
@@ -895,7 +920,8 @@ __device__ __forceinline__ ItemRange packed_piece(const PartialArgs& a, const Pa
   r.len = len;
   r.p_begin = max(g - st, 0);
   r.p_end = min(g_end, st + np) - st;  // <= p_begin: the item ends in the gap
-  r.n_valid = (st + np - 1) / pb.P - st / pb.P + 1;
+  // One split: the sequence lies within this item.
+  r.n_valid = st >= item * pb.P && st + np <= (item + 1) * pb.P ? 1 : 2;
   r.slot0 = item + b;
   r.g_end = st + r.p_end;
   r.paired = 0;
@@ -997,7 +1023,7 @@ __device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView
   PackedBatch& pb = w.pb;
   w.paired = false;
   if (!is_balanced(a.pages_per_split)) {
-    const int seq = item / a.num_splits;
+    const int seq = item / a.by_splits;
     load_first_ids<D>(a, seq, (item - seq * a.num_splits) * a.pages_per_split, first_id);
     w.it = fixed_item(a, item);
     make_uniform(w.it);
@@ -1048,7 +1074,7 @@ __device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView
       w.item_end = (item >> 1) * 2 * pb.P + ((item & 1) ? 2 * pb.P : pb.P + d);
     }
     g0 = __builtin_amdgcn_readfirstlane(g0);
-    const int b0 = min(g0 / P, a.batch - 1);
+    const int b0 = min(g0 / a.by_spec_pages, a.batch - 1);
     load_first_ids<D>(a, b0, g0 - b0 * P, first_id);
     if (!w.paired) load_lengths(a, pb.len);
     bool differs = false;
@@ -1193,7 +1219,7 @@ __device__ __forceinline__ void write_results(const PartialArgs& a, WaveState<NB
         const int rs = e / CPR;
         if (map.real(nb, rs)) {
           const int r = map.row(nb, rs);
-          const int qi = r / a.group;
+          const int qi = r / a.by_group;
           const int gg = r - qi * a.group;
           _Float16* op = a.out + ((size_t)(b * a.q_len + qi) * a.hq +
                                   map.head(nb, rs) * a.group + gg) * HD + 4 * (e % CPR);
@@ -1321,7 +1347,8 @@ struct StagedBits {
   const unsigned* words;
   bool masked;            // the caller's words; else the causal chain
   bool two;               // two words per row
-  int group, l16;
+  FastDiv by_group;
+  int l16;
   WaveRows<NB, HPW> map;
   __device__ __forceinline__ void get(unsigned long long (&dbits)[NB]) const {
 #pragma unroll
@@ -1330,7 +1357,7 @@ struct StagedBits {
         dbits[nb] = words[32 * nb + l16];
         if (two) dbits[nb] |= (unsigned long long)words[32 * nb + 16 + l16] << 32;
       } else {
-        const int qi = map.row(nb, l16) / group;
+        const int qi = map.row(nb, l16) / by_group;
         dbits[nb] = qi >= 63 ? ~0ull : (2ull << qi) - 1ull;
       }
     }
@@ -1368,7 +1395,9 @@ void sqa_partial_kernel(PartialArgs a) {
   // dependent trips through the scalar cache.
   asm volatile("" ::"s"(a.block_tables), "s"(a.seq_lens), "s"(a.batch), "s"(a.hkv),
                "s"(a.num_splits), "s"(a.pages_per_split), "s"(a.bt_stride), "s"(a.max_pages),
-               "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.hg_items[0]));
+               "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.hg_items[0]),
+               "s"(a.by_head_groups.mul), "s"(a.by_head_groups.shift), "s"(a.by_splits.mul),
+               "s"(a.by_splits.shift));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // blockIdx.x = item * head_groups + head_group, or with items per head group
@@ -1377,8 +1406,9 @@ void sqa_partial_kernel(PartialArgs a) {
   const bool hg_split = a.hg_items[0] > 0;
   const HeadGroupItems hgi =
       head_group_items(a.hg_items, a.batch, a.spec_pps, a.hg_spec_pps1, blockIdx.x);
-  const int hgrp = hg_split ? hgi.group : (int)blockIdx.x % head_groups;
-  const int item = hg_split ? hgi.item : (int)blockIdx.x / head_groups;
+  const int whole = (int)blockIdx.x / a.by_head_groups;
+  const int hgrp = hg_split ? hgi.group : (int)blockIdx.x - whole * head_groups;
+  const int item = hg_split ? hgi.item : whole;
   const PlanView view = hg_split ? plan_view(a, hgi) : plan_view(a);
   const int slot_heads = hg_split ? WW : a.hkv;  // partial slot layout (write_results)
   const int head0 = hg_split ? hgrp * WW : 0;
@@ -1445,7 +1475,7 @@ void sqa_partial_kernel(PartialArgs a) {
     for (int nb = 0; nb < NB; ++nb) {
       const int r = map.row(nb, tl);
       const bool real = map.real(nb, tl);
-      const int qi = real ? r / a.group : 0;
+      const int qi = real ? r / a.by_group : 0;
       const int gg = real ? r - qi * a.group : 0;
       const int hh = (real ? map.head(nb, tl) : map.kvh) * a.group + gg;
       const _Float16* qp = a.q + ((size_t)(b * a.q_len + qi) * a.hq + hh) * HD;
@@ -1459,7 +1489,7 @@ void sqa_partial_kernel(PartialArgs a) {
       for (int i = 0; i < kBitsLds / 64; ++i) {
         // Lane t fills dword 64 i + t: block nb, word w, row slot r.
         const int nb = min(2 * i + (t >> 5), NB - 1), w = (t >> 4) & 1;
-        const int qi = map.real(nb, tl) ? map.row(nb, tl) / a.group : 0;
+        const int qi = map.real(nb, tl) ? map.row(nb, tl) / a.by_group : 0;
         copy4_to_lds(a.draft_mask + (size_t)(b * a.q_len + qi) * a.mask_words +
                          (a.mask_words > 1 ? w : 0),
                      (unsigned)(size_t)(my_bits + buf * kBitsLds + 64 * i));
@@ -1567,7 +1597,7 @@ void sqa_partial_kernel(PartialArgs a) {
   wait_vmcnt_fence<D * HPW * KV::kLoads>();
   const u4* q_lds = my_q + (buf % kQBufs) * kQLds;
   const StagedBits<NB, HPW> bits{my_bits + buf * kBitsLds, a.draft_mask != nullptr,
-                                 a.mask_words > 1, a.group, l16, map};
+                                 a.mask_words > 1, a.by_group, l16, map};
   // Pages holding a token >= mask_from (draft block or past the end) are masked.
   const int mask_from = len - a.q_len;
 
@@ -1865,6 +1895,12 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   constexpr int kLoads = kSlot / (512 * 16);        // loads per thread and page
   constexpr int kThreads = 512;
   static_assert(HD * KV::kBytes == 16 * L::kChunks, "a token row is kChunks 16-byte chunks");
+  // As in sqa_partial_kernel: one round trip for the arguments.
+  asm volatile("" ::"s"(a.block_tables), "s"(a.seq_lens), "s"(a.batch), "s"(a.hkv),
+               "s"(a.num_splits), "s"(a.pages_per_split), "s"(a.bt_stride), "s"(a.max_pages),
+               "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.pair_items),
+               "s"(a.by_head_groups.mul), "s"(a.by_head_groups.shift), "s"(a.by_splits.mul),
+               "s"(a.by_splits.shift));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // blockIdx.x = item * head_groups + head_group; with paired items (two head
@@ -1873,8 +1909,9 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   // head slot.
   const int head_groups = (a.hkv + 3) / 4;
   const bool pairs = a.pair_items != 0;
-  const int hgrp = pairs ? (blockIdx.x & 3) >> 1 : blockIdx.x % head_groups;
-  const int item = pairs ? (blockIdx.x >> 2) * 2 + (blockIdx.x & 1) : blockIdx.x / head_groups;
+  const int whole = (int)blockIdx.x / a.by_head_groups;
+  const int hgrp = pairs ? (blockIdx.x & 3) >> 1 : blockIdx.x - whole * head_groups;
+  const int item = pairs ? (blockIdx.x >> 2) * 2 + (blockIdx.x & 1) : whole;
   const int hs = wave & 3;
   const int kvh = hgrp * 4 + hs;
   const HalfRows map{kvh, a.rows, a.hkv, 32 * (wave >> 2)};
@@ -1938,7 +1975,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   for (int nb = 0; nb < NB; ++nb) {
     const int r = map.row(nb, l16);
     const bool real = map.real(nb, l16);
-    const int qi = real ? r / a.group : 0;
+    const int qi = real ? r / a.by_group : 0;
     const int gg = real ? r - qi * a.group : 0;
     const int hh = real ? kvh * a.group + gg : 0;
     const _Float16* qp = a.q + ((size_t)(b * a.q_len + qi) * a.hq + hh) * HD;
@@ -2147,19 +2184,29 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   constexpr int SG = TPR / CH;      // split groups of a row
   constexpr int RPW = 256 / TPR;    // rows per workgroup
   static_assert(SG >= 1 && TPR % CH == 0 && 256 % TPR == 0, "a row's threads must cover its dims");
+  // The arguments in one round trip, as in sqa_partial_kernel.
+  asm volatile("" ::"s"(a.part_o), "s"(a.part_ml), "s"(a.seq_splits), "s"(a.batch), "s"(a.q_len),
+               "s"(a.hq), "s"(a.hkv), "s"(a.group), "s"(a.rows), "s"(a.pages_per_split),
+               "s"(a.num_splits), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.hg_items[0]),
+               "s"(a.by_hq.mul), "s"(a.by_hq.shift), "s"(a.by_seq_rows.mul),
+               "s"(a.by_seq_rows.shift), "s"(a.by_group.mul), "s"(a.by_group.shift),
+               "s"(a.by_spec_pps.mul), "s"(a.by_spec_pps.shift), "s"(a.tune), "s"(a.out),
+               "s"(a.out_scale));
   const int t = threadIdx.x;
   const int tr = t % TPR;
   const int c = tr % CH;
   const int g = tr / CH;
-  const int row = blockIdx.x * RPW + t / TPR;
+  // A row's threads are whole waves: everything about the row is uniform.
+  const int row = blockIdx.x * RPW + __builtin_amdgcn_readfirstlane(t / TPR);
   const int total = a.batch * a.q_len * a.hq;
   const bool live = row < total;  // uniform per row
   if (a.tune != nullptr && blockIdx.x == 0) update_pair_delta(a.tune, a.tune_records);
   const int rowc = live ? row : 0;
-  const int h = rowc % a.hq;
-  const int qi = (rowc / a.hq) % a.q_len;
-  const int b = rowc / (a.hq * a.q_len);
-  const int kvh = h / a.group;
+  const int b = rowc / a.by_seq_rows;
+  const int row_of_seq = rowc - b * a.q_len * a.hq;
+  const int qi = row_of_seq / a.by_hq;
+  const int h = row_of_seq - qi * a.hq;
+  const int kvh = h / a.by_group;
   const int r = qi * a.group + (h - kvh * a.group);
 
   // Where the row's splits are. Fixed plan: all num_splits slots of the
@@ -2178,7 +2225,7 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   const int grp = kvh >> 2;
   const int num_splits = hg_split ? a.hg_items[grp] + a.batch : a.num_splits;
   const SeqSplits* seq_splits = a.seq_splits + (hg_split ? grp * a.batch : 0);
-  const int spec_pps = hg_split && grp ? a.hg_spec_pps1 : a.spec_pps;
+  const FastDiv by_spec_pps = hg_split && grp ? a.by_spec_pps1 : a.by_spec_pps;
   // items between consecutive splits of this row, and the row's item in split 0
   const size_t stride = (size_t)(hg_split ? 4 : a.hkv) * a.rows;
   const size_t row_item =
@@ -2188,8 +2235,8 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   SeqSplits table = {0, 0};
   if (expect) {
     const int start = b * a.spec_pages;
-    const int i0 = start / spec_pps;
-    n_valid = (start + a.spec_pages - 1) / spec_pps - i0 + 1;
+    const int i0 = start / by_spec_pps;
+    n_valid = (start + a.spec_pages - 1) / by_spec_pps - i0 + 1;
     slot0 = i0 + b;
   } else if (balanced) {
     table = in_range(seq_splits[b], num_splits);
@@ -2302,14 +2349,34 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
     for (int i = 0; i < DPT; ++i) acc[i] = acc[i] * sa + ao[i] * so;
     mt = nm;
   };
-#pragma unroll
-  for (int off = CH; off < 64; off <<= 1) {
-    const float mo = __shfl_xor(mt, off), dn = __shfl_xor(den, off);
+  static_assert(CH >= 8, "split groups of a wave meet over 8, 16 and 32 lanes");
+  if constexpr (CH <= 8) {
+    // Lanes l and l ^ 8 of a row of 16: a rotation by 8.
+    auto other = [](float x) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+          0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false));  // row_ror:8
+    };
+    const float mo = other(mt), dn = other(den);
     float ao[DPT];
 #pragma unroll
-    for (int i = 0; i < DPT; ++i) ao[i] = __shfl_xor(acc[i], off);
+    for (int i = 0; i < DPT; ++i) ao[i] = other(acc[i]);
     combine(mo, dn, ao);
   }
+  auto meet = [&](auto pair_of) {
+    const LanePair m2 = pair_of(mt), d2 = pair_of(den);
+    float ao[DPT];
+    mt = m2.lo;
+    den = d2.lo;
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) {
+      const LanePair a2 = pair_of(acc[i]);
+      acc[i] = a2.lo;
+      ao[i] = a2.hi;
+    }
+    combine(m2.hi, d2.hi, ao);
+  };
+  if constexpr (CH <= 16) meet([](float x) { return lane_pair<16>(x); });
+  if constexpr (CH <= 32) meet([](float x) { return lane_pair<32>(x); });
   if constexpr (WPR > 1) {
     static_assert(RPW == 1, "the LDS combine serves one row per workgroup");
     __shared__ float sm_acc[WPR][CH][DPT + 1];
