@@ -57,7 +57,10 @@ extern "C" {
  *     max_seq_len > 0 it is -P, P = ceil(max_seq_len / 16) (at most max_pages):
  *     the kernels first assume every sequence spans P pages, which saves a
  *     memory round trip when it holds, and verify it (the result is the same
- *     either way). Otherwise a fixed plan as above.
+ *     either way). Otherwise a fixed plan as above. A call whose sequences are
+ *     short (P pages, or the whole table row, in splits of a few pages) cuts
+ *     every sequence from its own start instead, as a fixed plan does, reading
+ *     the same pages.
  * max_pages: 16-token pages a block-table row addresses (block_tables columns
  * x page_size / 16); num_splits and pages_per_split count 16-token pages too.
  * max_seq_len <= 0 means "unknown": a fixed plan covers max_pages * 16 tokens.
@@ -97,11 +100,12 @@ size_t sqa_workspace_bytes(int batch, int q_len, int num_query_heads, int num_kv
  * 4-byte (SQA_ERR_INVALID otherwise), and a plan's partial sums must stay within
  * 0xFFFF0000 bytes (SQA_ERR_INVALID; the automatic plans need a few MB to ~40 MB).
  * Allocates nothing and never synchronises.
- * A fixed plan (pages_per_split > 0) says which pages are read: the first
- * num_splits * pages_per_split of every sequence. Where the given workspace also
- * holds the automatic plan over those pages and that plan is the faster cut, the
- * call runs it instead (the sums then round in another order; the same arguments
- * and workspace size give the same bits). A workspace of that size, that is the
+ * A plan says which pages are read: a fixed one (pages_per_split > 0) the first
+ * num_splits * pages_per_split of every sequence, a balanced one all. Where the
+ * given workspace also holds the automatic plan over a fixed plan's pages and that
+ * is the faster cut, the call runs it instead, and a balanced plan over short
+ * sequences is cut at their starts (the sums then round in another order; the same
+ * arguments and workspace size give the same bits). A workspace of that size, that is the
  * larger of sqa_workspace_bytes for the two plans, lets a few sequences in coarse
  * chunks use the whole chip; one of the fixed plan's own size is always enough.
  * `timing_events`: NULL, or an array of 3 hipEvent_t recorded on `stream`

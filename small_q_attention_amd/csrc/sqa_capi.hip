@@ -58,6 +58,14 @@ int fixed_plan(int batch, int num_kv_heads, long long pages, long long pps, int*
   return SQA_OK;
 }
 
+// Work items that fill the chip once: one wave of resident workgroups, shared by
+// the head groups.
+long long wave_items(int cus, long long rows, int num_kv_heads, int head_dim) {
+  const sqa::LaunchShape sh = sqa::launch_shape((int)rows, num_kv_heads, head_dim);
+  const long long head_groups = (num_kv_heads + sh.heads - 1) / sh.heads;
+  return ceil_div((long long)cus * sh.wg_per_cu, head_groups);
+}
+
 // The automatic plan (sqa_plan_splits with chunk_keys 0) over `pages` pages per
 // sequence; `known`: no sequence spans more.
 int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int head_dim,
@@ -65,10 +73,7 @@ int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int 
                    int* pages_per_split) {
   int cus = sqa_device_cu_count(device);
   if (cus <= 0) return SQA_ERR_HIP;
-  // One wave of resident workgroups over the whole chip.
-  const sqa::LaunchShape sh = sqa::launch_shape((int)rows, num_kv_heads, head_dim);
-  const long long head_groups = (num_kv_heads + sh.heads - 1) / sh.heads;
-  const long long slots_target = ceil_div((long long)cus * sh.wg_per_cu, head_groups);
+  const long long slots_target = wave_items(cus, rows, num_kv_heads, head_dim);
   if (batch > 1 && batch <= sqa::kMaxBalancedBatch) {
     // Balanced plan: the kernel sizes splits from the batch's total pages,
     // so ragged batches keep every workgroup equally busy. The slot count
@@ -101,65 +106,114 @@ int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int 
   return fixed_plan(batch, num_kv_heads, pages, pps, num_splits, pages_per_split);
 }
 
-// What a call with a fixed plan runs. The plan says which pages of every
-// sequence are read (the first num_splits * pages_per_split); how they are cut
-// changes only the order of the sums. Chunks of a caller's choosing (the
-// reference's default is 512 keys) leave most of the chip idle for a few
-// sequences (one of 8K keys: 32 workgroups on 256 CUs) and run a second,
-// partly filled wave of workgroups for many. So the same pages are cut as the
-// automatic plan cuts them, where the caller's workspace holds that plan:
-// *num_splits and *pages_per_split are replaced, and the pages a sequence may
-// span returned (kernel_pages unchanged without a re-cut).
-//
+// How a call cuts the pages of its plan.
+struct Cut {
+  int num_splits, pages_per_split;
+  long long pages;  // kernel pages of a sequence the call may read
+  bool open_end;    // fixed: the last split of a sequence runs to its end
+};
+
+// Short sequences: a balanced item of a few pages spans sequence ends, and every
+// piece of it and every merged row costs as much as the pages. So where each
+// sequence's own share of the wave's items, `per_seq`, cuts its pages into splits
+// of at most kShortSplitPages (or into one of kShortSinglePages: no partials, no
+// merge kernel), the splits start with the sequences: a fixed plan. Whole calls,
+// balanced -> fixed, fp16, head dim 128, q_len 4: 4 sequences of 200 keys 15.5 ->
+// 11.4 us, 8 of 1.5K 17.2 -> 14.3, 64 ragged of up to 100 keys 26.9 -> 10.5; q_len
+// 16, 32 of 512, 28.9 -> 28.4. Over 1368 shapes of 2-250 sequences of 100-8K keys,
+// uniform and ragged, the rule took 996 calls to the fixed cut, 1.24x in the
+// geometric mean, the slowest 0.98x; with 16 pages for 12 ragged batches lose up
+// to 15%, as the balanced items then spread what the longest sequence holds.
+constexpr long long kShortSplitPages = 12, kShortSinglePages = 32;
+bool short_cut(long long items, int batch, int num_kv_heads, long long pages,
+               long long kernel_pages, Cut* cut) {
+  const long long per_seq = std::max(1LL, items / batch);
+  // Splits of an even number of pages: lengths expected a page or two apart (a
+  // caller's longest length and its table's width) mostly get the same cut, so the
+  // same bits.
+  long long want = std::max(ceil_div(pages, per_seq), (long long)sqa::kMinSplitPages);
+  if (per_seq > 1) want += want & 1;
+  int ns = 0, pps = 0;
+  if (fixed_plan(batch, num_kv_heads, pages, want, &ns, &pps) != SQA_OK) return false;
+  if (pps > (ns > 1 ? kShortSplitPages : kShortSinglePages)) return false;
+  // Open-ended, the last split holds what a sequence longer than expected has left.
+  if (cut->open_end && kernel_pages - (long long)(ns - 1) * pps > sqa::kMaxSplitPages)
+    return false;
+  cut->num_splits = ns;
+  cut->pages_per_split = pps;
+  return true;
+}
+
+// What a call runs. A plan says which pages of every sequence are read (a fixed
+// one the first num_splits * pages_per_split, a balanced one all); how they are
+// cut changes only the order of the sums. A balanced plan of at least a wave of
+// items over short sequences takes short_cut(). A fixed plan of a caller's chunk
+// size (the reference's default is 512 keys) leaves most of the chip idle for a
+// few sequences (one of 8K keys: 32 workgroups on 256 CUs) and runs a second,
+// partly filled wave of workgroups for many: the same pages are cut as the
+// automatic plan (and short_cut) would, where the caller's workspace holds that.
 // Measured with 512-key chunks, as given -> re-cut (us per call, back to back):
 // one sequence of 8K keys 35.2 -> 13.7 (q_len 2), of 32K keys 46.1 -> 28.4; two
 // of 8K keys, q_len 8, 43.6 -> 23.9. Kept as given:
 // - plans past kMaxBalancedBatch sequences (the automatic plan is then another
 //   fixed one);
 // - several sequences whose splits come to more than a quarter of a wave of
-//   work items (an eighth past 32 rows) and less than four waves: there a balanced item that spans a
-//   sequence end costs as much as the idle workgroups (64 ragged sequences of
-//   up to 1K keys, q_len 8: 49 as given, 68 re-cut), while four waves of
-//   start-ups cost 4-70%;
+//   work items (an eighth past 32 rows) and less than four waves: there a
+//   balanced item that spans a sequence end costs as much as the idle workgroups
+//   (64 ragged sequences of up to 1K keys, q_len 8: 49 as given, 68 re-cut),
+//   while four waves of start-ups cost 4-70%;
 // - one split per sequence (no partials, no merge kernel) unless an item gets
 //   shorter by kMinPagesSaved pages, and, for several sequences, by twice that
 //   with at most 1/16 of a wave of items (200 keys, 8 sequences: 15 us as given,
 //   17 re-cut; 512 keys: 32 and 15).
 constexpr int kMinPagesSaved = 12;
-long long recut_plan(const sqa_attention_args& a, long long rows, long long kernel_pages,
-                     int* num_splits, int* pages_per_split) {
-  if (sqa::is_balanced(*pages_per_split) || a.batch > sqa::kMaxBalancedBatch || !a.workspace ||
-      (uintptr_t)a.workspace % 16)
-    return kernel_pages;
-  const long long cover = std::min((long long)*num_splits * *pages_per_split, kernel_pages);
-  if (cover >= (1LL << 24) || a.batch * cover >= (1LL << 30)) return kernel_pages;
-  int device = -1, ns = 0, pps = 0;
-  if (hipGetDevice(&device) != hipSuccess ||
-      automatic_plan(device, a.batch, rows, a.num_kv_heads, a.head_dim, cover, (int)cover, true,
-                     &ns, &pps) != SQA_OK)
-    return kernel_pages;
-  const long long item = sqa::is_balanced(pps)
-                             ? sqa::packed_item_pages((int)(a.batch * cover), ns - a.batch)
-                             : pps;
-  const long long given = (long long)a.batch * *num_splits;
-  if (a.batch > 1) {
-    const long long wave = ns - a.batch;  // items of the balanced plan
-    if (*num_splits > 1 ? (rows > 32 ? 8 : 4) * given > wave && given < 4 * wave
-                        : 16 * given > wave)
-      return kernel_pages;
+Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_pages) {
+  const Cut as_given{a.num_splits, a.pages_per_split, kernel_pages, false};
+  const bool balanced = sqa::is_balanced(a.pages_per_split);
+  if (a.batch > sqa::kMaxBalancedBatch || !a.workspace || (uintptr_t)a.workspace % 16 ||
+      (a.flags & SQA_FLAG_ADAPTIVE_PAIRS))
+    return as_given;
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess) return as_given;
+  const int cus = sqa_device_cu_count(device);
+  if (cus <= 0) return as_given;
+  const long long wave = wave_items(cus, rows, a.num_kv_heads, a.head_dim);
+  Cut cut = as_given;
+  if (balanced) {
+    if (a.batch < 2 || a.num_splits - a.batch < wave) return as_given;
+    const int expected = sqa::spec_pages_of(a.pages_per_split);
+    cut.open_end = true;
+    if (!short_cut(wave, a.batch, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
+                   kernel_pages, &cut))
+      return as_given;
+  } else {
+    cut.pages = std::min((long long)a.num_splits * a.pages_per_split, kernel_pages);
+    if (cut.pages >= (1LL << 24) || a.batch * cut.pages >= (1LL << 30) ||
+        automatic_plan(device, a.batch, rows, a.num_kv_heads, a.head_dim, cut.pages,
+                       (int)cut.pages, true, &cut.num_splits, &cut.pages_per_split) != SQA_OK)
+      return as_given;
+    const long long given = (long long)a.batch * a.num_splits;
+    if (a.batch > 1 &&
+        (a.num_splits > 1 ? (rows > 32 ? 8 : 4) * given > wave && given < 4 * wave
+                          : 16 * given > wave))
+      return as_given;
+    if (a.batch > 1)
+      short_cut(wave, a.batch, a.num_kv_heads, cut.pages, cut.pages, &cut);
+    const long long item =
+        sqa::is_balanced(cut.pages_per_split)
+            ? sqa::packed_item_pages((int)(a.batch * cut.pages), cut.num_splits - a.batch)
+            : cut.pages_per_split;
+    if (a.num_splits == 1 && cut.pages - item < (a.batch > 1 ? 2 : 1) * kMinPagesSaved)
+      return as_given;
   }
-  if (*num_splits == 1 && cover - item < (a.batch > 1 ? 2 : 1) * kMinPagesSaved)
-    return kernel_pages;
   const unsigned long long part_o_bytes =
-      (unsigned long long)sqa::plan_slots(a.batch, ns, pps) * a.num_kv_heads * rows * a.head_dim *
-      sizeof(float);
+      (unsigned long long)sqa::plan_slots(a.batch, cut.num_splits, cut.pages_per_split) *
+      a.num_kv_heads * rows * a.head_dim * sizeof(float);
   if (part_o_bytes > sqa::kMaxPartialBytes ||
-      sqa_workspace_bytes(a.batch, a.q_len, a.num_query_heads, a.num_kv_heads, a.head_dim, ns,
-                          pps) > a.workspace_bytes)
-    return kernel_pages;
-  *num_splits = ns;
-  *pages_per_split = pps;
-  return cover;
+      sqa_workspace_bytes(a.batch, a.q_len, a.num_query_heads, a.num_kv_heads, a.head_dim,
+                          cut.num_splits, cut.pages_per_split) > a.workspace_bytes)
+    return as_given;
+  return cut;
 }
 
 }  // namespace
@@ -355,7 +409,9 @@ int run_attention(const sqa_attention_args& a) {
   if ((balanced || num_splits > 1) && part_o_bytes > sqa::kMaxPartialBytes)
     return fail(SQA_ERR_INVALID, "the plan's partials (%llu bytes) exceed %llu bytes",
                 part_o_bytes, sqa::kMaxPartialBytes);
-  const long long call_pages = recut_plan(a, rows, kernel_pages, &num_splits, &pages_per_split);
+  const Cut cut = cut_for_call(a, rows, kernel_pages);
+  num_splits = cut.num_splits;
+  pages_per_split = cut.pages_per_split;
   balanced = sqa::is_balanced(pages_per_split);
   spec_pages = sqa::spec_pages_of(pages_per_split);
   part_o_bytes = partial_bytes();
@@ -393,7 +449,8 @@ int run_attention(const sqa_attention_args& a) {
   pa.head_dim = head_dim;
   pa.bt_stride = max_pages;
   pa.page_shift = page_shift;
-  pa.max_pages = (int)call_pages;
+  pa.max_pages = (int)cut.pages;
+  pa.open_end = cut.open_end;
   pa.pages_per_split = balanced ? 0 : pages_per_split;
   pa.num_splits = num_splits;
   pa.spec_pages = spec_pages;
@@ -476,7 +533,7 @@ int run_attention(const sqa_attention_args& a) {
     ma.group = group;
     ma.rows = (int)rows;
     ma.head_dim = head_dim;
-    ma.max_pages = (int)call_pages;
+    ma.max_pages = (int)cut.pages;
     ma.pages_per_split = pa.pages_per_split;
     ma.num_splits = num_splits;
     ma.spec_pages = spec_pages;

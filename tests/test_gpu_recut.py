@@ -74,3 +74,26 @@ def test_a_recut_plan_reads_the_pages_of_the_plan_as_given(batch, splits, pps):
     for out, label in ((as_given, "as given"), (recut, "re-cut")):
         assert_parity(out[:, :1].contiguous(), want, label=label)
     assert (as_given.float() - recut.float()).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("q_len", [2, 8, 16])
+@pytest.mark.parametrize("lens,promise,width", [
+    ([100] * 2, 100, 7), ([0, 1, 17, 190, 33], 190, 12), ([400] * 40, 400, 25),
+    ([31 * (i % 16) for i in range(130)], 465, 32), ([90, 5, 0, 64] * 64, 90, 6),
+    # Longer than promised: the last split runs on to the sequence's end.
+    ([700, 90, 3000, 16, 0, 1], 128, 200),
+    # A table whose rows hold more than a split may: not cut, the promise broken too.
+    ([700, 90, 3000, 16, 0, 1], 128, 2300),
+    ([700, 90, 300, 16, 0, 1], 0, 44),  # no promise: the table's width
+])
+def test_short_sequences_are_cut_at_their_starts(q_len, lens, promise, width):
+    case = inputs.Case(batch=len(lens), q_len=q_len, seq_lens=lens, seed=2400 + q_len)
+    q, k, v, bt, sl = inputs.make_inputs(case)
+    wide = torch.zeros(len(lens), width, dtype=torch.int32)
+    wide[:, :bt.shape[1]] = bt
+    ref = attention_c64(q, k, v, bt, sl, 16, 8)
+    dev = tuple(t.cuda() for t in (q, k, v, wide, sl))
+    for given in {promise, 0}:
+        out = sqa.paged_mtp_attention(*dev, 16, given)
+        assert_parity(out, ref, label=f"q{q_len} B{len(lens)} promise {given}")
+        assert torch.equal(out, sqa.paged_mtp_attention(*dev, 16, given))
