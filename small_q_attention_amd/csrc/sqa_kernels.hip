@@ -2096,7 +2096,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
 // with l_s <= 0 are skipped and a row with no visible key is written as 0.
 // fp16 partials hold acc_s / l_s (so acc_s = l_s times the stored row).
 //
-// One pass, every load of a round in flight at once: WPR waves serve one
+// One pass, every load of a round in flight at once: TPR threads serve one
 // output row; each thread owns the 16 bytes of a partial row at dims DPT c ..
 // DPT c + DPT - 1 (DPT = 8 fp16 or 4 fp32 values) and the splits g, g + SG, ...
 // of its split group g, U splits per round (one round wherever the row's
@@ -2173,18 +2173,19 @@ __device__ __noinline__ void update_pair_delta(float* tune, int records) {
   if (t == 0) tune[2] = 0.f;
 }
 
-template <int WPR, int HD, typename E, int U>
+template <int TPR, int HD, typename E, int U>
 __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   // Each thread owns DPT dims of the row, 16 bytes of every partial row (fp16
   // partials: 8 dims; fp32: 4), and the splits g, g + SG, ... of its split
-  // group g; a row's WPR waves cover SG = 64 WPR / CH splits per load
+  // group g; a row's TPR threads cover SG = TPR / CH splits per load
   // instruction and U SG splits per round.
   constexpr int DPT = E::kHalfPartials ? 8 : 4;
   constexpr int CH = HD / DPT;      // threads per partial row
-  constexpr int TPR = 64 * WPR;     // threads per output row
   constexpr int SG = TPR / CH;      // split groups of a row
+  constexpr int WPR = TPR / 64;     // waves of a row (0: several rows per wave)
   constexpr int RPW = 256 / TPR;    // rows per workgroup
   static_assert(SG >= 1 && TPR % CH == 0 && 256 % TPR == 0, "a row's threads must cover its dims");
+  static_assert(SG == 1 || WPR >= 1, "split groups meet within whole waves");
   // The arguments in one round trip, as in sqa_partial_kernel.
   asm volatile("" ::"s"(a.part_o), "s"(a.part_ml), "s"(a.seq_splits), "s"(a.batch), "s"(a.q_len),
                "s"(a.hq), "s"(a.hkv), "s"(a.group), "s"(a.rows), "s"(a.pages_per_split),
@@ -2197,8 +2198,9 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   const int tr = t % TPR;
   const int c = tr % CH;
   const int g = tr / CH;
-  // A row's threads are whole waves: everything about the row is uniform.
-  const int row = blockIdx.x * RPW + __builtin_amdgcn_readfirstlane(t / TPR);
+  // Where a row's threads are whole waves everything about the row is uniform.
+  const int row =
+      blockIdx.x * RPW + (WPR >= 1 ? __builtin_amdgcn_readfirstlane(t / TPR) : t / TPR);
   const int total = a.batch * a.q_len * a.hq;
   const bool live = row < total;  // uniform per row
   if (a.tune != nullptr && blockIdx.x == 0) update_pair_delta(a.tune, a.tune_records);
@@ -2351,7 +2353,7 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
     mt = nm;
   };
   static_assert(CH >= 8, "split groups of a wave meet over 8, 16 and 32 lanes");
-  if constexpr (CH <= 8) {
+  if constexpr (SG > 1 && CH <= 8) {
     // Lanes l and l ^ 8 of a row of 16: a rotation by 8.
     auto other = [](float x) {
       return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
@@ -2376,8 +2378,8 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
     }
     combine(m2.hi, d2.hi, ao);
   };
-  if constexpr (CH <= 16) meet([](float x) { return lane_pair<16>(x); });
-  if constexpr (CH <= 32) meet([](float x) { return lane_pair<32>(x); });
+  if constexpr (SG > 1 && CH <= 16) meet([](float x) { return lane_pair<16>(x); });
+  if constexpr (SG > 1 && CH <= 32) meet([](float x) { return lane_pair<32>(x); });
   if constexpr (WPR > 1) {
     static_assert(RPW == 1, "the LDS combine serves one row per workgroup");
     __shared__ float sm_acc[WPR][CH][DPT + 1];
@@ -2493,32 +2495,50 @@ void launch_partial_as(const PartialArgs& a, const LaunchShape& sh, dim3 grid, d
     launch_partial_hd<128, E, KV<128>>(a, sh, grid, block, stream);
 }
 
-template <int HD, typename E, int WPR>
-void launch_merge_u(const MergeArgs& a, int u, dim3 grid, hipStream_t stream) {
+template <int HD, typename E, int TPR>
+void launch_merge_u(const MergeArgs& a, int u, hipStream_t stream) {
+  constexpr int kRows = 256 / TPR;  // per workgroup
+  const dim3 grid((unsigned)((a.batch * a.q_len * a.hq + kRows - 1) / kRows));
   if (u <= 2)
-    hipLaunchKernelGGL((sqa_merge_kernel<WPR, HD, E, 2>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 2>), grid, dim3(256), 0, stream, a);
   else if (u <= 4)
-    hipLaunchKernelGGL((sqa_merge_kernel<WPR, HD, E, 4>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 4>), grid, dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((sqa_merge_kernel<WPR, HD, E, 8>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 8>), grid, dim3(256), 0, stream, a);
 }
 
 template <int HD, typename E>
 void launch_merge_hd(const MergeArgs& a, int per_row, hipStream_t stream) {
-  // A row's splits in one round of loads wherever 8 per thread cover them: a
-  // wave per row (4 rows per workgroup) for 1024 rows and more, where the
-  // chip has rows enough; a workgroup of 4 waves per row below that, or where a
-  // wave would need a second round (one sequence, KV 32K, q_len 8: 128 splits
-  // per row). Each thread issues U loads of 16 bytes at once, the smallest U of
-  // 2, 4, 8 that covers the row (more rounds past 8).
-  constexpr int kSplitsPerWave = 64 / (HD / (E::kHalfPartials ? 8 : 4));
+  // Three ways to share a row's splits, each thread issuing U loads of 16 bytes at
+  // once (the smallest U of 2, 4, 8 that covers the row; more rounds past 8):
+  // - the threads of one partial row take all of the row's splits, several rows per
+  //   wave and no exchange between lanes: up to 8 splits per row where the rows
+  //   still come to two waves per SIMD. A wave per row leaves most of its lanes
+  //   without a split there and takes four times the waves (whole calls, wave per
+  //   row -> this: 64 short ragged sequences, q_len 4, 58.0 -> 55.9 us; 64 of 512
+  //   keys, q_len 16, 45.1 -> 36.6; 128 of up to 1K, q_len 8, 78.8 -> 67.2). At
+  //   half as many rows the two are even (16 of 8K, q_len 8: 87.9 and 87.4) or the
+  //   wave per row is ahead (16 of up to 2K, q_len 8: 27.5 and 28.1);
+  // - a wave per row (4 rows per workgroup) from 1024 rows on, wherever 8 loads per
+  //   thread cover the row's splits;
+  // - a workgroup of 4 waves per row below that, or where a wave would need a
+  //   second round (one sequence, KV 32K, q_len 8: 128 splits per row).
+  constexpr int kChunks = HD / (E::kHalfPartials ? 8 : 4);  // threads a partial row takes
+  constexpr int kSplitsPerWave = 64 / kChunks;
+  constexpr long long kManyThreads = 256 * 4 * 2 * 64;
   const int total = a.batch * a.q_len * a.hq;
+  if constexpr (kChunks < 64) {
+    if ((long long)total * kChunks >= kManyThreads && per_row <= 8) {
+      launch_merge_u<HD, E, kChunks>(a, per_row, stream);
+      return;
+    }
+  }
   if (total >= 1024 && per_row <= 8 * kSplitsPerWave) {
     const int u = (per_row + kSplitsPerWave - 1) / kSplitsPerWave;
-    launch_merge_u<HD, E, 1>(a, u, dim3((unsigned)((total + 3) / 4)), stream);
+    launch_merge_u<HD, E, 64>(a, u, stream);
   } else {
     const int u = (per_row + 4 * kSplitsPerWave - 1) / (4 * kSplitsPerWave);
-    launch_merge_u<HD, E, 4>(a, u, dim3((unsigned)total), stream);
+    launch_merge_u<HD, E, 256>(a, u, stream);
   }
 }
 
