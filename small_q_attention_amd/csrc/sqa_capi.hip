@@ -116,26 +116,38 @@ struct Cut {
 // Short sequences: a balanced item of a few pages spans sequence ends, and every
 // piece of it and every merged row costs as much as the pages. So where each
 // sequence's own share of the wave's items, `per_seq`, cuts its pages into splits
-// of at most kShortSplitPages (or into one of kShortSinglePages: no partials, no
-// merge kernel), the splits start with the sequences: a fixed plan. Whole calls,
-// balanced -> fixed, fp16, head dim 128, q_len 4: 4 sequences of 200 keys 15.5 ->
-// 11.4 us, 8 of 1.5K 17.2 -> 14.3, 64 ragged of up to 100 keys 26.9 -> 10.5; q_len
-// 16, 32 of 512, 28.9 -> 28.4. Over 1368 shapes of 2-250 sequences of 100-8K keys,
-// uniform and ragged, the rule took 996 calls to the fixed cut, 1.24x in the
-// geometric mean, the slowest 0.98x; with 16 pages for 12 ragged batches lose up
-// to 15%, as the balanced items then spread what the longest sequence holds.
-constexpr long long kShortSplitPages = 12, kShortSinglePages = 32;
-bool short_cut(long long items, int batch, int num_kv_heads, long long pages,
+// of at most kShortSplitPages, the splits start with the sequences: a fixed plan.
+// Whole calls, balanced -> fixed, fp16, head dim 128, q_len 4: 4 sequences of 200
+// keys 15.5 -> 11.4 us, 8 of 1.5K 17.2 -> 14.3, 64 ragged of up to 100 keys 26.9 ->
+// 10.5. Over 1368 shapes of 2-250 sequences of 100-8K keys, uniform and ragged,
+// the rule took 996 calls to the fixed cut, 1.24x in the geometric mean, the
+// slowest 0.98x; with 16 pages for 12 ragged batches lose up to 15%, as the
+// balanced items then spread what the longest sequence holds.
+// One split per sequence needs no partials and no merge kernel. It wins up to
+// kSoloPages wherever there is more than one to choose from (7 pages: 1.0-1.4x,
+// but 0.92x past 32 rows for a few sequences, whose 64-row splits are shared by
+// more CUs), and up to kShortSinglePages where a sequence has one item to itself
+// (32 pages, 128 sequences: 1.1-1.6x, of them ragged), or two of more than 32 rows,
+// whose partial rows cost most (64 of 32 pages, q_len 16: 1.3x).
+constexpr long long kShortSplitPages = 12, kSoloPages = 8, kShortSinglePages = 32;
+bool short_cut(long long items, int batch, long long rows, int num_kv_heads, long long pages,
                long long kernel_pages, Cut* cut) {
   const long long per_seq = std::max(1LL, items / batch);
+  const long long solo = per_seq == 1 || (per_seq == 2 && rows > 32) ? kShortSinglePages
+                         : rows <= 32 || per_seq <= 4                ? kSoloPages
+                                                                     : sqa::kMinSplitPages;
   // Splits of an even number of pages: lengths expected a page or two apart (a
   // caller's longest length and its table's width) mostly get the same cut, so the
   // same bits.
   long long want = std::max(ceil_div(pages, per_seq), (long long)sqa::kMinSplitPages);
-  if (per_seq > 1) want += want & 1;
+  want += want & 1;
+  if (pages <= solo)
+    want = pages;
+  else if (batch == 1)
+    return false;  // the automatic plan is a fixed one
   int ns = 0, pps = 0;
   if (fixed_plan(batch, num_kv_heads, pages, want, &ns, &pps) != SQA_OK) return false;
-  if (pps > (ns > 1 ? kShortSplitPages : kShortSinglePages)) return false;
+  if (ns == 1 ? pages > solo : pps > kShortSplitPages) return false;
   // Open-ended, the last split holds what a sequence longer than expected has left.
   if (cut->open_end && kernel_pages - (long long)(ns - 1) * pps > sqa::kMaxSplitPages)
     return false;
@@ -154,19 +166,16 @@ bool short_cut(long long items, int batch, int num_kv_heads, long long pages,
 // automatic plan (and short_cut) would, where the caller's workspace holds that.
 // Measured with 512-key chunks, as given -> re-cut (us per call, back to back):
 // one sequence of 8K keys 35.2 -> 13.7 (q_len 2), of 32K keys 46.1 -> 28.4; two
-// of 8K keys, q_len 8, 43.6 -> 23.9. Kept as given:
-// - plans past kMaxBalancedBatch sequences (the automatic plan is then another
-//   fixed one);
-// - several sequences whose splits come to more than a quarter of a wave of
-//   work items (an eighth past 32 rows) and less than four waves: there a
-//   balanced item that spans a sequence end costs as much as the idle workgroups
-//   (64 ragged sequences of up to 1K keys, q_len 8: 49 as given, 68 re-cut),
-//   while four waves of start-ups cost 4-70%;
-// - one split per sequence (no partials, no merge kernel) unless an item gets
-//   shorter by kMinPagesSaved pages, and, for several sequences, by twice that
-//   with at most 1/16 of a wave of items (200 keys, 8 sequences: 15 us as given,
-//   17 re-cut; 512 keys: 32 and 15).
-constexpr int kMinPagesSaved = 12;
+// of 8K keys, q_len 8, 43.6 -> 23.9. Kept as given: plans past kMaxBalancedBatch
+// sequences (the automatic plan is then another fixed one); one split per sequence
+// (no partials, no merge) under kMinRecutPages, or where the cut would be a
+// balanced one; and, where it would be, chunks that come to between half a wave and
+// two or three waves of work items (an eighth past 32 rows, whose partial rows cost
+// most, or with many sequences): there balanced items that span sequence ends lose
+// more than idle or late workgroups do (937 shapes; 64 ragged sequences of up to 1K
+// keys, q_len 16, 2 splits each: 43 us as given, 76 balanced), while past two waves
+// the start-ups cost 7-40%.
+constexpr long long kMinRecutPages = 16;
 Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_pages) {
   const Cut as_given{a.num_splits, a.pages_per_split, kernel_pages, false};
   const bool balanced = sqa::is_balanced(a.pages_per_split);
@@ -183,7 +192,7 @@ Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_p
     if (a.batch < 2 || a.num_splits - a.batch < wave) return as_given;
     const int expected = sqa::spec_pages_of(a.pages_per_split);
     cut.open_end = true;
-    if (!short_cut(wave, a.batch, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
+    if (!short_cut(wave, a.batch, rows, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
                    kernel_pages, &cut))
       return as_given;
   } else {
@@ -192,19 +201,19 @@ Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_p
         automatic_plan(device, a.batch, rows, a.num_kv_heads, a.head_dim, cut.pages,
                        (int)cut.pages, true, &cut.num_splits, &cut.pages_per_split) != SQA_OK)
       return as_given;
+    const bool shorter =
+        short_cut(wave, a.batch, rows, a.num_kv_heads, cut.pages, cut.pages, &cut);
     const long long given = (long long)a.batch * a.num_splits;
-    if (a.batch > 1 &&
-        (a.num_splits > 1 ? (rows > 32 ? 8 : 4) * given > wave && given < 4 * wave
-                          : 16 * given > wave))
-      return as_given;
-    if (a.batch > 1)
-      short_cut(wave, a.batch, a.num_kv_heads, cut.pages, cut.pages, &cut);
-    const long long item =
-        sqa::is_balanced(cut.pages_per_split)
-            ? sqa::packed_item_pages((int)(a.batch * cut.pages), cut.num_splits - a.batch)
-            : cut.pages_per_split;
-    if (a.num_splits == 1 && cut.pages - item < (a.batch > 1 ? 2 : 1) * kMinPagesSaved)
-      return as_given;
+    bool better;
+    if (a.num_splits == 1)
+      better = (shorter || a.batch == 1) && cut.pages >= kMinRecutPages;
+    else if (a.batch == 1 || shorter)
+      better = true;
+    else if (given < wave)
+      better = rows > 32 ? 8 * given <= wave : 2 * given <= wave && 8 * a.batch <= wave;
+    else
+      better = given >= 3 * wave || (given >= 2 * wave && 4 * a.batch <= wave);
+    if (!better) return as_given;
   }
   const unsigned long long part_o_bytes =
       (unsigned long long)sqa::plan_slots(a.batch, cut.num_splits, cut.pages_per_split) *
