@@ -1016,14 +1016,14 @@ __device__ __forceinline__ bool piece_at(const PartialArgs& a, ItemWalk& w, int 
 // sequence spec_pages pages, item size spec_pps from the host) the plan needs no
 // lengths, so the ids go out with them, and a length that does not match falls
 // back to the plan from the loaded lengths.
-// kPairs: paired items may be asked for.
-template <int D, bool kPairs>
+// kPairs: paired items may be asked for; kBalanced: the plan is a balanced one.
+template <int D, bool kPairs, bool kBalanced>
 __device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView& v, int item,
                                             ItemWalk& w, int (&first_id)[D]) {
   const int lane = threadIdx.x & 63;
   PackedBatch& pb = w.pb;
   w.paired = false;
-  if (!is_balanced(a.pages_per_split)) {
+  if constexpr (!kBalanced) {
     const int seq = item / a.by_splits;
     load_first_ids<D>(a, seq, (item - seq * a.num_splits) * a.pages_per_split, first_id);
     w.it = fixed_item(a, item);
@@ -1031,7 +1031,7 @@ __device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView
     w.item_end = 1;
     w.g_end = 1;
     return w.it.b >= 0;
-  }
+  } else {
   bool ids_loaded = false;
   int g = 0;
   if (a.spec_pages > 0) {
@@ -1102,22 +1102,22 @@ __device__ __forceinline__ bool first_piece(const PartialArgs& a, const PlanView
   if (!piece_at(a, w, item, g)) return false;  // uniform
   if (!ids_loaded) load_first_ids<D>(a, w.it.b, w.it.p_begin, first_id);
   return true;
+  }
 }
 
 // Runs `piece(range, first_id)` for every piece of workgroup item `item`.
 // Consecutive pieces are separated by a barrier (they reuse the workgroup's LDS).
 // Returns whether the item ran as a paired item (every workgroup of a call
 // returns the same).
-template <int D, typename Piece>
+template <int D, bool kBalanced, typename Piece>
 __device__ __forceinline__ bool for_each_piece(const PartialArgs& a, const PlanView& v, int item,
                                                Piece&& piece) {
-  const bool balanced = is_balanced(a.pages_per_split);
   int first_id[D];
   ItemWalk w;
-  bool more = first_piece<D, true>(a, v, item, w, first_id);
+  bool more = first_piece<D, true, kBalanced>(a, v, item, w, first_id);
   while (more) {  // uniform
     piece(w.it, first_id);
-    more = balanced && piece_at(a, w, item, w.it.g_end);
+    more = kBalanced && piece_at(a, w, item, w.it.g_end);
     if (more) {
       load_first_ids<D>(a, w.it.b, w.it.p_begin, first_id);
       __syncthreads();  // the previous piece is done with the LDS
@@ -1376,6 +1376,12 @@ struct StagedBits {
 // softmax state and writes its own partials (or, with a single split, the
 // output). Every K/V byte is read by one wave only, so the loads are
 // non-temporal.
+// The two kinds of plan are instantiations of their own (BAL: balanced), here and in
+// the merge kernel: a call of a few pages runs almost every instruction for the
+// first time, and the way to its first load led around the other plan's code (per
+// call, one kernel for both -> each its own: one sequence of 1K keys, q_len 2, 10.2
+// -> 9.3 us; of 8K, q_len 4, 13.85 -> 13.2, q_len 8 17.7 -> 16.7; of 4K, q_len 16,
+// 18.7 -> 17.3; long calls +-0.3%).
 // The page ring runs through the pieces of an item: the next piece's first pages
 // are requested in this one's last turn and its Q and mask words as soon as this
 // one begins, so a sequence end costs the epilogue (about 1 us) and not a drained
@@ -1386,7 +1392,7 @@ struct StagedBits {
 // nine page ids for every piece, now one for the item). Long uniform batches, whose
 // items end with their sequences, are unchanged. What bounds it: HBM, and for few
 // pages per item the start-up.
-template <int NB, int D, int WW, int WPE, int HD, typename E, typename KV, int HPW,
+template <int NB, int D, int WW, int WPE, int HD, typename E, typename KV, int HPW, bool BAL,
           bool RB = false>
 __global__ __launch_bounds__(WW * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void sqa_partial_kernel(PartialArgs a) {
@@ -1404,7 +1410,7 @@ void sqa_partial_kernel(PartialArgs a) {
   // blockIdx.x = item * head_groups + head_group, or with items per head group
   // (hg_items) as head_group_items() deals them.
   const int head_groups = (a.hkv + WW * HPW - 1) / (WW * HPW);
-  const bool hg_split = a.hg_items[0] > 0;
+  const bool hg_split = BAL && a.hg_items[0] > 0;
   const HeadGroupItems hgi =
       head_group_items(a.hg_items, a.batch, a.spec_pps, a.hg_spec_pps1, blockIdx.x);
   const int whole = (int)blockIdx.x / a.by_head_groups;
@@ -1420,7 +1426,7 @@ void sqa_partial_kernel(PartialArgs a) {
   const bool active = kvh < a.hkv;
   const WaveRows<NB, HPW> map{kvh, a.rows, a.hkv};
 
-  const bool balanced = is_balanced(a.pages_per_split);
+  constexpr bool balanced = BAL;  // the plan; its code only
   const bool single = !balanced && a.num_splits == 1;  // no merge kernel follows
 
   // The page loop of each of the three forms below (see there).
@@ -1449,7 +1455,7 @@ void sqa_partial_kernel(PartialArgs a) {
   // The first piece of the item and the ids of its first D pages, requested.
   ItemWalk walk;
   int first_id[D];
-  if (!first_piece<D, false>(a, view, item, walk, first_id)) return;  // uniform
+  if (!first_piece<D, false, BAL>(a, view, item, walk, first_id)) return;  // uniform
   ItemRange it = walk.it;
   const size_t first_slot = (size_t)it.slot0 + it.split;
   if (it.p_begin >= it.p_end && !single) {  // fixed plan only
@@ -1886,7 +1892,7 @@ struct LdsSlice<KvNative<128>> {
 // 0.3% faster for fp16 and 3.8% for bf16 at KV 32K x 16 sequences. Pages past the
 // split load through a zero-length resource (zeros, no memory traffic), as in
 // sqa_partial_kernel.
-template <int D, typename E, typename KV>
+template <int D, typename E, typename KV, bool BAL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 void sqa_partial_lds_kernel(PartialArgs a) {
   constexpr int HD = 128, NB = 2, KK = Dims<HD>::KK, MB = Dims<HD>::MB;
@@ -1909,7 +1915,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   // workgroups of an item run on XCDs of the item's parity. wave = half * 4 +
   // head slot.
   const int head_groups = (a.hkv + 3) / 4;
-  const bool pairs = a.pair_items != 0;
+  const bool pairs = BAL && a.pair_items != 0;
   const int whole = (int)blockIdx.x / a.by_head_groups;
   const int hgrp = pairs ? (blockIdx.x & 3) >> 1 : blockIdx.x - whole * head_groups;
   const int item = pairs ? (blockIdx.x >> 2) * 2 + (blockIdx.x & 1) : whole;
@@ -1920,7 +1926,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   // and meet the barriers; they skip the math.
   const bool active = kvh < a.hkv && map.base < a.rows;
 
-  const bool balanced = is_balanced(a.pages_per_split);
+  constexpr bool balanced = BAL;
   const bool single = !balanced && a.num_splits == 1;
   static_assert(D + 1 <= kIdPad, "page-id table padding must cover the ring's look-ahead");
   constexpr int kIdSlots = (kMaxSplitPages + kIdPad + kThreads - 1) / kThreads;
@@ -1948,7 +1954,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   float loop_ticks = 0.f;
   int loop_pages = 0;
   const bool paired_call =
-      for_each_piece<D>(a, plan_view(a), item, [&](const ItemRange& it, const int (&first_id)[D]) {
+      for_each_piece<D, BAL>(a, plan_view(a), item, [&](const ItemRange& it, const int (&first_id)[D]) {
   const int tid = piece_tid();
   const int lane = tid & 63;
   const int g16 = lane >> 4;
@@ -2083,7 +2089,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
   // from every workgroup. Whenever adaptive pairing was asked for, workgroup 0
   // stamps the call (or clears the stamp when the lengths made it fall back):
   // the merge kernel reads the records only under a stamp of this call.
-  if (a.pair_items == kPairsAdaptive && threadIdx.x == 0) {
+  if (BAL && a.pair_items == kPairsAdaptive && threadIdx.x == 0) {
     if (paired_call)
       *(int2*)(a.tune + 4 + 2 * blockIdx.x) =
           int2{__float_as_int(loop_ticks), loop_pages | (item & 1) << 30 | 1 << 31};
@@ -2178,7 +2184,7 @@ struct Count {
   static constexpr int value = N;
 };
 
-template <int TPR, int HD, typename E, int U>
+template <int TPR, int HD, typename E, int U, bool BAL>
 __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   // Each thread owns DPT dims of the row, 16 bytes of every partial row (fp16
   // partials: 8 dims; fp32: 4), and the splits g, g + SG, ... of its split
@@ -2211,7 +2217,7 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
                : (t / TPR) * gridDim.x + blockIdx.x;
   const int total = a.batch * a.q_len * a.hq;
   const bool live = row < total;  // uniform per row
-  if (a.tune != nullptr && blockIdx.x == 0) update_pair_delta(a.tune, a.tune_records);
+  if (BAL && a.tune != nullptr && blockIdx.x == 0) update_pair_delta(a.tune, a.tune_records);
   const int rowc = live ? row : 0;
   const int b = rowc / a.by_seq_rows;
   const int row_of_seq = rowc - b * a.q_len * a.hq;
@@ -2228,11 +2234,11 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
   // (sequence b's pages from b * spec_pages on, items of spec_pps pages) is
   // assumed while the table is read, and the row is merged again from the
   // table if the two differ.
-  const bool balanced = is_balanced(a.pages_per_split);
+  constexpr bool balanced = BAL;
   const bool expect = balanced && a.spec_pages > 0;
   // With items per head group (hg_items) the row's head group has its own
   // region of slots (four kv heads each), table, slot count and item size.
-  const bool hg_split = a.hg_items[0] > 0;
+  const bool hg_split = BAL && a.hg_items[0] > 0;
   const int grp = kvh >> 2;
   const int num_splits = hg_split ? a.hg_items[grp] + a.batch : a.num_splits;
   const SeqSplits* seq_splits = a.seq_splits + (hg_split ? grp * a.batch : 0);
@@ -2453,7 +2459,7 @@ __global__ __launch_bounds__(256) void sqa_merge_kernel(MergeArgs a) {
 // us, q16 278 (6 pages) -> 261 (3) -> 251 us (2); head dim 256 q8 342.7 ->
 // 325.1 us; head dim 64 q4 / q8 / q16 104.2 / 119.8 / 185 -> 100.7 / 116.6 /
 // 169 us (2 pages at 64 rows there lose the pipelined loop: 154 -> 165 us).
-template <int HD, typename E, typename KV>
+template <int HD, typename E, typename KV, bool BAL>
 void launch_partial_hd(const PartialArgs& a, const LaunchShape& sh, dim3 grid, dim3 block,
                        hipStream_t stream) {
   constexpr int D4 = 4 * 128 / HD, D2 = 2 * 128 / HD;
@@ -2466,71 +2472,71 @@ void launch_partial_hd(const PartialArgs& a, const LaunchShape& sh, dim3 grid, d
     // Two heads per wave: half the pages in flight, each twice the bytes.
     if constexpr (HD == 64) {
       if (sh.row_blocks == 1)
-        hipLaunchKernelGGL((sqa_partial_kernel<1, D2, 4, 1, HD, E, KV, 2>), grid, block, 0,
+        hipLaunchKernelGGL((sqa_partial_kernel<1, D2, 4, 1, HD, E, KV, 2, BAL>), grid, block, 0,
                            stream, a);
       else if (sh.row_blocks == 2)
-        hipLaunchKernelGGL((sqa_partial_kernel<2, D2, 4, 1, HD, E, KV, 2>), grid, block, 0,
+        hipLaunchKernelGGL((sqa_partial_kernel<2, D2, 4, 1, HD, E, KV, 2, BAL>), grid, block, 0,
                            stream, a);
       else
-        hipLaunchKernelGGL((sqa_partial_kernel<4, D2, 4, 1, HD, E, KV, 2>), grid, block, 0,
+        hipLaunchKernelGGL((sqa_partial_kernel<4, D2, 4, 1, HD, E, KV, 2, BAL>), grid, block, 0,
                            stream, a);
     }
   } else if (sh.row_blocks == 1) {
     if constexpr (HD == 128 && KV::kBytes == 2) {
       if (a.ring_batch) {
-        hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, true>), grid, block, 0,
+        hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block, 0,
                            stream, a);
         return;
       }
     }
-    hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1>), grid, block, 0, stream,
+    hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, BAL>), grid, block, 0, stream,
                        a);
   } else if (sh.row_blocks == 2) {
     if constexpr (HD == 128 && KV::kBytes == 2) {
       if (a.ring_batch) {
-        hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1, true>), grid, block, 0,
+        hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block, 0,
                            stream, a);
         return;
       }
     }
-    hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1>), grid, block, 0, stream,
+    hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1, BAL>), grid, block, 0, stream,
                        a);
   } else if constexpr (HD == 128 && KV::kBytes == 2) {
     // 33..64 rows of 16-bit K and V: two waves per kv head sharing an LDS ring
     // of 128 KiB (4 pages). e4m3 caches take the one-wave-per-head kernel below:
     // it widens each page once per head where two waves would both widen it
     // (cfg3 shape q16: 256.3 -> 246.6 us; B4 KV 8K 34.8 -> 33.6 us).
-    hipLaunchKernelGGL((sqa_partial_lds_kernel<4, E, KV>), grid, dim3(512), 0, stream, a);
+    hipLaunchKernelGGL((sqa_partial_lds_kernel<4, E, KV, BAL>), grid, dim3(512), 0, stream, a);
   } else if constexpr (HD != 256) {
-    hipLaunchKernelGGL((sqa_partial_kernel<4, D3, 4, 1, HD, E, KV, 1>), grid, block, 0, stream,
+    hipLaunchKernelGGL((sqa_partial_kernel<4, D3, 4, 1, HD, E, KV, 1, BAL>), grid, block, 0, stream,
                        a);
   }
 }
 
-template <typename E, template <int> class KV>
+template <typename E, template <int> class KV, bool BAL>
 void launch_partial_as(const PartialArgs& a, const LaunchShape& sh, dim3 grid, dim3 block,
                        hipStream_t stream) {
   if (a.head_dim == 64)
-    launch_partial_hd<64, E, KV<64>>(a, sh, grid, block, stream);
+    launch_partial_hd<64, E, KV<64>, BAL>(a, sh, grid, block, stream);
   else if (a.head_dim == 256)
-    launch_partial_hd<256, E, KV<256>>(a, sh, grid, block, stream);
+    launch_partial_hd<256, E, KV<256>, BAL>(a, sh, grid, block, stream);
   else
-    launch_partial_hd<128, E, KV<128>>(a, sh, grid, block, stream);
+    launch_partial_hd<128, E, KV<128>, BAL>(a, sh, grid, block, stream);
 }
 
-template <int HD, typename E, int TPR>
+template <int HD, typename E, int TPR, bool BAL>
 void launch_merge_u(const MergeArgs& a, int u, hipStream_t stream) {
   constexpr int kRows = 256 / TPR;  // per workgroup
   const dim3 grid((unsigned)((a.batch * a.q_len * a.hq + kRows - 1) / kRows));
   if (u <= 2)
-    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 2>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 2, BAL>), grid, dim3(256), 0, stream, a);
   else if (u <= 4)
-    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 4>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 4, BAL>), grid, dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 8>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((sqa_merge_kernel<TPR, HD, E, 8, BAL>), grid, dim3(256), 0, stream, a);
 }
 
-template <int HD, typename E>
+template <int HD, typename E, bool BAL>
 void launch_merge_hd(const MergeArgs& a, int per_row, hipStream_t stream) {
   // Three ways to share a row's splits, each thread issuing U loads of 16 bytes at
   // once (the smallest U of 2, 4, 8 that covers the row; more rounds past 8):
@@ -2552,27 +2558,51 @@ void launch_merge_hd(const MergeArgs& a, int per_row, hipStream_t stream) {
   const int total = a.batch * a.q_len * a.hq;
   if constexpr (kChunks < 64) {
     if ((long long)total * kChunks >= kManyThreads && per_row <= 8) {
-      launch_merge_u<HD, E, kChunks>(a, per_row, stream);
+      launch_merge_u<HD, E, kChunks, BAL>(a, per_row, stream);
       return;
     }
   }
   if (total >= 1024 && per_row <= 8 * kSplitsPerWave) {
     const int u = (per_row + kSplitsPerWave - 1) / kSplitsPerWave;
-    launch_merge_u<HD, E, 64>(a, u, stream);
+    launch_merge_u<HD, E, 64, BAL>(a, u, stream);
   } else {
     const int u = (per_row + 4 * kSplitsPerWave - 1) / (4 * kSplitsPerWave);
-    launch_merge_u<HD, E, 256>(a, u, stream);
+    launch_merge_u<HD, E, 256, BAL>(a, u, stream);
   }
 }
 
-template <typename E>
+template <typename E, bool BAL>
 void launch_merge_as(const MergeArgs& a, int per_row, hipStream_t stream) {
   if (a.head_dim == 64)
-    launch_merge_hd<64, E>(a, per_row, stream);
+    launch_merge_hd<64, E, BAL>(a, per_row, stream);
   else if (a.head_dim == 256)
-    launch_merge_hd<256, E>(a, per_row, stream);
+    launch_merge_hd<256, E, BAL>(a, per_row, stream);
   else
-    launch_merge_hd<128, E>(a, per_row, stream);
+    launch_merge_hd<128, E, BAL>(a, per_row, stream);
+}
+
+template <bool BAL>
+void launch_partial_plan(const PartialArgs& a, const LaunchShape& sh, dim3 grid, dim3 block,
+                         hipStream_t stream) {
+  if (a.bf16) {
+    if (a.kv_fp8)
+      launch_partial_as<ElemBF16, KvFp8, BAL>(a, sh, grid, block, stream);
+    else
+      launch_partial_as<ElemBF16, KvNative, BAL>(a, sh, grid, block, stream);
+  } else {
+    if (a.kv_fp8)
+      launch_partial_as<ElemF16, KvFp8, BAL>(a, sh, grid, block, stream);
+    else
+      launch_partial_as<ElemF16, KvNative, BAL>(a, sh, grid, block, stream);
+  }
+}
+
+template <bool BAL>
+void launch_merge_plan(const MergeArgs& a, int per_row, hipStream_t stream) {
+  if (a.bf16)
+    launch_merge_as<ElemBF16, BAL>(a, per_row, stream);
+  else
+    launch_merge_as<ElemF16, BAL>(a, per_row, stream);
 }
 
 }  // namespace
@@ -2587,17 +2617,10 @@ hipError_t launch_partial(const PartialArgs& a, hipStream_t stream) {
                               : (long long)a.batch * a.num_splits;
   const dim3 grid((unsigned)(items * head_groups));
   const dim3 block(sh.waves() * 64);
-  if (a.bf16) {
-    if (a.kv_fp8)
-      launch_partial_as<ElemBF16, KvFp8>(a, sh, grid, block, stream);
-    else
-      launch_partial_as<ElemBF16, KvNative>(a, sh, grid, block, stream);
-  } else {
-    if (a.kv_fp8)
-      launch_partial_as<ElemF16, KvFp8>(a, sh, grid, block, stream);
-    else
-      launch_partial_as<ElemF16, KvNative>(a, sh, grid, block, stream);
-  }
+  if (is_balanced(a.pages_per_split))
+    launch_partial_plan<true>(a, sh, grid, block, stream);
+  else
+    launch_partial_plan<false>(a, sh, grid, block, stream);
   return hipGetLastError();
 }
 
@@ -2613,10 +2636,10 @@ hipError_t launch_merge(const MergeArgs& a, hipStream_t stream) {
   const int items = a.hg_items[0] > 0 ? max(a.hg_items[0], a.hg_items[1]) : a.num_splits - a.batch;
   const int per_row = is_balanced(a.pages_per_split) ? (items + a.batch - 1) / a.batch
                                                      : a.num_splits;
-  if (a.bf16)
-    launch_merge_as<ElemBF16>(a, per_row, stream);
+  if (is_balanced(a.pages_per_split))
+    launch_merge_plan<true>(a, per_row, stream);
   else
-    launch_merge_as<ElemF16>(a, per_row, stream);
+    launch_merge_plan<false>(a, per_row, stream);
   return hipGetLastError();
 }
 
