@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import struct
 import threading
 from pathlib import Path
 
@@ -59,6 +60,10 @@ class AttentionArgs(ctypes.Structure):
                 ("timing_events", _C.c_void_p), ("dtype", _C.c_int), ("kv_dtype", _C.c_int),
                 ("flags", _C.c_int)]
 
+
+# AttentionArgs as one packed record (native sizes and alignment, padded as C does).
+_ARGS = struct.Struct("@N2P2P4q2PiPi2f8iPN2P3i0q")
+assert _ARGS.size == ctypes.sizeof(AttentionArgs)
 
 DTYPE_F16, DTYPE_BF16, DTYPE_FP8_E4M3 = 0, 1, 2
 FLAG_ADAPTIVE_PAIRS = 1  # SQA_FLAG_ADAPTIVE_PAIRS
@@ -197,51 +202,43 @@ def launch(query, key_cache, value_cache, block_tables, seq_lens, output, worksp
         raise RuntimeError(f"sqa_paged_mtp_attention failed: {last_error(lib)}")
 
 
-def kv_cache(k_view, v_view) -> KVCache:
-    """Describe a paged cache from two ``[num_pages, page, Hkv, D]`` views of any strides
-    (separate caches, or the K / V halves of an interleaved NHD or HND cache). The head
-    dimension must be contiguous and K and V must share strides."""
-    if k_view.dim() != 4 or v_view.shape != k_view.shape:
-        raise ValueError("K and V views must both be [num_pages, page, Hkv, D]")
-    if k_view.stride() != v_view.stride() or k_view.stride(3) != 1:
-        raise ValueError("K and V views must share strides with a contiguous head dimension")
-    return KVCache(k_view.data_ptr(), v_view.data_ptr(), k_view.shape[0], k_view.stride(0),
-                   k_view.stride(1), k_view.stride(2))
-
-
 def launch_general(query, output, k_view, v_view, block_tables, seq_lens, draft_mask,
                    scale: float, out_scale: float, num_splits: int, pages_per_split: int,
                    workspace, stream_handle: int, timing_events=None, flags: int = 0):
     """Call ``sqa_paged_attention``. ``query``/``output``: contiguous ``[B, Q, Hq, D]``;
-    ``k_view``/``v_view``: see :func:`kv_cache`; ``draft_mask``: ``None`` (causal draft
+    ``k_view``/``v_view``: ``[num_pages, page, Hkv, D]`` views of equal strides with a
+    contiguous head dimension (separate caches, or the K / V halves of an interleaved NHD
+    or HND cache); ``draft_mask``: ``None`` (causal draft
     chain) or a contiguous 32-bit ``[B, Q, W]`` tensor of packed draft bits; ``flags``:
     0 or :data:`FLAG_ADAPTIVE_PAIRS`."""
+    import torch
+
     lib = _LIB if _LIB is not None else load()
     b, q_len, hq, d = query.shape
-    a = AttentionArgs()
-    a.struct_size = ctypes.sizeof(AttentionArgs)
-    a.query, a.output = query.data_ptr(), output.data_ptr()
-    a.kv = kv_cache(k_view, v_view)
-    a.block_tables, a.seq_lens = block_tables.data_ptr(), seq_lens.data_ptr()
-    a.max_pages = block_tables.shape[1]
-    if draft_mask is not None:
-        a.draft_mask, a.mask_words = draft_mask.data_ptr(), draft_mask.shape[-1]
-    a.scale, a.out_scale = float(scale), float(out_scale)
-    a.batch, a.q_len, a.num_query_heads, a.num_kv_heads = b, q_len, hq, k_view.shape[2]
-    a.head_dim, a.page_size = d, k_view.shape[1]
-    a.num_splits, a.pages_per_split = num_splits, pages_per_split
-    if workspace is not None:
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = workspace.numel() * workspace.element_size()
-    a.stream = stream_handle
-    a.dtype = DTYPE_BF16 if str(query.dtype) == "torch.bfloat16" else DTYPE_F16
-    a.kv_dtype = DTYPE_FP8_E4M3 if str(k_view.dtype) == "torch.float8_e4m3fn" else a.dtype
-    a.flags = int(flags)
+    if k_view.dim() != 4 or v_view.shape != k_view.shape:
+        raise ValueError("K and V views must both be [num_pages, page, Hkv, D]")
+    strides = k_view.stride()
+    if strides != v_view.stride() or strides[3] != 1:
+        raise ValueError("K and V views must share strides with a contiguous head dimension")
+    num_pages, page, hkv, _ = k_view.shape
+    words, mask_words = (0, 0) if draft_mask is None else (draft_mask.data_ptr(),
+                                                           draft_mask.shape[-1])
+    ws, ws_bytes = (0, 0) if workspace is None else (
+        workspace.data_ptr(), workspace.numel() * workspace.element_size())
+    dtype = DTYPE_BF16 if query.dtype is torch.bfloat16 else DTYPE_F16
+    kv_dtype = (DTYPE_FP8_E4M3
+                if k_view.dtype is getattr(torch, "float8_e4m3fn", None) else dtype)
     ev = None
     if timing_events is not None:
         ev = (ctypes.c_void_p * 3)(*[ctypes.c_void_p(int(e)) for e in timing_events])
-        a.timing_events = ctypes.cast(ev, ctypes.c_void_p)
-    rc = lib.sqa_paged_attention(ctypes.byref(a))
+    # Every field at once: assigning them one by one took 4 us of a call.
+    a = _ARGS.pack(
+        _ARGS.size, query.data_ptr(), output.data_ptr(), k_view.data_ptr(), v_view.data_ptr(),
+        num_pages, strides[0], strides[1], strides[2], block_tables.data_ptr(),
+        seq_lens.data_ptr(), block_tables.shape[1], words, mask_words, scale, out_scale, b, q_len,
+        hq, hkv, d, page, num_splits, pages_per_split, ws, ws_bytes, stream_handle or 0,
+        0 if ev is None else ctypes.addressof(ev), dtype, kv_dtype, flags)
+    rc = lib.sqa_paged_attention(a)
     if rc != SQA_OK:
         raise RuntimeError(f"sqa_paged_attention failed: {last_error(lib)}")
 
