@@ -237,7 +237,7 @@ def launch_general(query, output, k_view, v_view, block_tables, seq_lens, draft_
         num_pages, strides[0], strides[1], strides[2], block_tables.data_ptr(),
         seq_lens.data_ptr(), block_tables.shape[1], words, mask_words, scale, out_scale, b, q_len,
         hq, hkv, d, page, num_splits, pages_per_split, ws, ws_bytes, stream_handle or 0,
-        0 if ev is None else ctypes.addressof(ev), dtype, kv_dtype, flags)
+        0 if ev is None else ctypes.addressof(ev), dtype, kv_dtype, int(flags))
     rc = lib.sqa_paged_attention(a)
     if rc != SQA_OK:
         raise RuntimeError(f"sqa_paged_attention failed: {last_error(lib)}")

@@ -245,3 +245,47 @@ def test_fp16_launcher_refuses_other_element_types(dtype):
     sl = torch.full((1,), 64, dtype=torch.int32)
     with pytest.raises(TypeError, match="launch_general"):
         _lib.launch(q, k, k, bt, sl, torch.empty_like(q), None, 1, 4, 0)
+
+
+class _Recorder:
+    """Stands in for the library: keeps the record ``sqa_paged_attention`` is given."""
+
+    def sqa_paged_attention(self, record):
+        self.args = _lib.AttentionArgs.from_buffer_copy(record)
+        return SQA_OK
+
+
+@pytest.mark.parametrize("scale, out_scale, flags", [
+    (0.125, 1.0, 0), (1e39, -1e39, 1), (float("inf"), 1e-46, 0), (1, 2, 1.0)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_general_launcher_fills_every_field_of_the_record(monkeypatch, scale, out_scale, flags,
+                                                          masked):
+    """The packed record against ``AttentionArgs`` assigned field by field; floats past
+    the float range become infinities, as in a C assignment."""
+    import torch
+
+    rec = _Recorder()
+    monkeypatch.setattr(_lib, "_LIB", rec)
+    q = torch.zeros(3, 2, 8, 64, dtype=torch.bfloat16)
+    out = torch.empty_like(q)
+    cache = torch.zeros(5, 2, 32, 4, 64, dtype=torch.float8_e4m3fn)
+    k, v = cache[:, 0], cache[:, 1]
+    bt, sl = torch.zeros(3, 7, dtype=torch.int32), torch.ones(3, dtype=torch.int32)
+    words = torch.zeros(3, 2, 1, dtype=torch.int32) if masked else None
+    ws = torch.zeros(1000, dtype=torch.float32)
+    _lib.launch_general(q, out, k, v, bt, sl, words, scale, out_scale, 6, -14, ws, 12345,
+                        flags=flags)
+    want = _lib.AttentionArgs(
+        struct_size=ctypes.sizeof(_lib.AttentionArgs), query=q.data_ptr(), output=out.data_ptr(),
+        kv=_lib.KVCache(k.data_ptr(), v.data_ptr(), 5, *k.stride()[:3]),
+        block_tables=bt.data_ptr(), seq_lens=sl.data_ptr(), max_pages=7,
+        draft_mask=words.data_ptr() if masked else None, mask_words=int(masked),
+        scale=float(scale), out_scale=float(out_scale), batch=3, q_len=2, num_query_heads=8,
+        num_kv_heads=4, head_dim=64, page_size=32, num_splits=6, pages_per_split=-14,
+        workspace=ws.data_ptr(), workspace_bytes=4000, stream=12345, dtype=_lib.DTYPE_BF16,
+        kv_dtype=_lib.DTYPE_FP8_E4M3, flags=int(flags))
+    for name, _ in _lib.AttentionArgs._fields_:
+        if name != "kv":
+            assert getattr(rec.args, name) == getattr(want, name), name
+    for name, _ in _lib.KVCache._fields_:
+        assert getattr(rec.args.kv, name) == getattr(want.kv, name), name
