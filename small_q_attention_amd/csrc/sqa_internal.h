@@ -278,9 +278,12 @@ constexpr int kRingPages = 4;
 
 // What a second piece costs a workgroup of the balanced plan, in pages of its
 // own: ~5.6 us measured at 16 ragged sequences of 2K-32K tokens (q_len 8, head
-// dim 128, fp16), where one page of the workgroup's (16 tokens of K and V for 4
-// kv heads, 32 KiB) takes ~1.15 us; scaled by the bytes of a workgroup's page
-// for other shapes and element types. The 8-wave LDS kernel (33..64 rows, head
+// dim 128, fp16) when the page ring was drained at a sequence end, where one page
+// of the workgroup's (16 tokens of K and V for 4 kv heads, 32 KiB) takes ~1.15 us.
+// With the ring running through the pieces 3 pages do as well or better by up to
+// 2.7% (64 sequences of up to 2K keys, q_len 4, 58.6 -> 57.0 us per call; 16 of
+// 2K-32K 176.7 -> 176.1), but the plan's layout is stated with 5. Scaled by the
+// bytes of a workgroup's page for other shapes and element types. The 8-wave LDS kernel (33..64 rows, head
 // dim 128, 16-bit K/V) restarts a ring behind a barrier per page and writes
 // 64 rows per head: 8 pages measured best there (ragged q16 fp16 190.2 -> 187.8
 // us, bf16 194.4 -> 190.2; 12 pages 187.8 / 190.8; with one barrier per page
