@@ -100,14 +100,9 @@ size_t sqa_workspace_bytes(int batch, int q_len, int num_query_heads, int num_kv
  * 4-byte (SQA_ERR_INVALID otherwise), and a plan's partial sums must stay within
  * 0xFFFF0000 bytes (SQA_ERR_INVALID; the automatic plans need a few MB to ~40 MB).
  * Allocates nothing and never synchronises.
- * A plan says which pages are read: a fixed one (pages_per_split > 0) the first
- * num_splits * pages_per_split of every sequence, a balanced one all. Where the
- * given workspace also holds the automatic plan over a fixed plan's pages and that
- * is the faster cut, the call runs it instead, and a balanced plan over short
- * sequences is cut at their starts (the sums then round in another order; the same
- * arguments and workspace size give the same bits). A workspace of that size, that is the
- * larger of sqa_workspace_bytes for the two plans, lets a few sequences in coarse
- * chunks use the whole chip; one of the fixed plan's own size is always enough.
+ * A fixed plan (pages_per_split > 0) reads the first num_splits * pages_per_split
+ * pages of every sequence in the splits it gives; a balanced plan reads all pages,
+ * and one over short sequences is cut at their starts (sqa_plan_splits).
  * `timing_events`: NULL, or an array of 3 hipEvent_t recorded on `stream`
  * before the partial kernel, between the two kernels and after the merge
  * kernel (used by the benchmark to time the partial kernel alone).

@@ -67,7 +67,6 @@ assert _ARGS.size == ctypes.sizeof(AttentionArgs)
 
 DTYPE_F16, DTYPE_BF16, DTYPE_FP8_E4M3 = 0, 1, 2
 FLAG_ADAPTIVE_PAIRS = 1  # SQA_FLAG_ADAPTIVE_PAIRS
-MAX_BALANCED_BATCH = 256  # sequences a balanced plan takes (kMaxBalancedBatch)
 
 
 def library_path() -> Path:
@@ -142,24 +141,6 @@ def workspace_bytes(batch: int, q_len: int, num_query_heads: int, num_kv_heads: 
     """Workspace of a plan from :func:`plan_splits` (``pages_per_split`` 0 = balanced)."""
     return int(load().sqa_workspace_bytes(batch, q_len, num_query_heads, num_kv_heads, head_dim,
                                           num_splits, pages_per_split))
-
-
-@functools.lru_cache(maxsize=4096)
-def call_workspace_bytes(device_index: int, batch: int, q_len: int, num_query_heads: int,
-                         num_kv_heads: int, head_dim: int, num_splits: int,
-                         pages_per_split: int, max_pages: int) -> int:
-    """Workspace handed to a call: the plan's own, and for a fixed plan (a caller's chunk
-    size) at least the automatic plan's over the same pages, which the library then
-    runs instead (``sqa_paged_mtp_attention``). ``max_pages`` counts 16-token pages."""
-    need = workspace_bytes(batch, q_len, num_query_heads, num_kv_heads, head_dim, num_splits,
-                           pages_per_split)
-    if pages_per_split > 0 and batch <= MAX_BALANCED_BATCH:
-        cover = min(num_splits * pages_per_split, max_pages)
-        auto = plan_splits(device_index, batch, q_len, num_query_heads, num_kv_heads, head_dim,
-                           min(cover * 16, 0x7fffffff), cover, 0)
-        need = max(need, workspace_bytes(batch, q_len, num_query_heads, num_kv_heads, head_dim,
-                                         *auto))
-    return need
 
 
 def raw_stream(device_index: int) -> int:
@@ -252,9 +233,7 @@ def run(query, key_cache, value_cache, block_tables, seq_lens, num_splits: int,
 
     out = torch.empty_like(query)
     b, q_len, hq, d = query.shape
-    nbytes = call_workspace_bytes(query.device.index or 0, b, q_len, hq, key_cache.shape[2], d,
-                                  num_splits, pages_per_split,
-                                  block_tables.shape[1] * (key_cache.shape[1] // 16))
+    nbytes = workspace_bytes(b, q_len, hq, key_cache.shape[2], d, num_splits, pages_per_split)
     stream = raw_stream(query.device.index)
     ws = workspace_for(nbytes, query, query.device.index, stream) if nbytes else None
     if query.dtype == torch.float16:
@@ -315,8 +294,8 @@ def run_fp16(query, key_cache, value_cache, block_tables, seq_lens, batch: int, 
     import torch
 
     out = torch.empty_like(query)
-    nbytes = call_workspace_bytes(device_index, batch, q_len, num_query_heads, num_kv_heads, 128,
-                                  num_splits, pages_per_split, max_pages * (page_size // 16))
+    nbytes = workspace_bytes(batch, q_len, num_query_heads, num_kv_heads, 128, num_splits,
+                             pages_per_split)
     stream = raw_stream(device_index)
     ws = workspace_for(nbytes, query, device_index, stream) if nbytes else None
     rc = _LIB.sqa_paged_mtp_attention(

@@ -109,8 +109,7 @@ int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int 
 // How a call cuts the pages of its plan.
 struct Cut {
   int num_splits, pages_per_split;
-  long long pages;  // kernel pages of a sequence the call may read
-  bool open_end;    // fixed: the last split of a sequence runs to its end
+  bool open_end;  // fixed: the last split of a sequence runs to its end
 };
 
 // Short sequences: a balanced item of a few pages spans sequence ends, and every
@@ -141,45 +140,26 @@ bool short_cut(long long items, int batch, long long rows, int num_kv_heads, lon
   // same bits.
   long long want = std::max(ceil_div(pages, per_seq), (long long)sqa::kMinSplitPages);
   want += want & 1;
-  if (pages <= solo)
-    want = pages;
-  else if (batch == 1)
-    return false;  // the automatic plan is a fixed one
+  if (pages <= solo) want = pages;
   int ns = 0, pps = 0;
   if (fixed_plan(batch, num_kv_heads, pages, want, &ns, &pps) != SQA_OK) return false;
   if (ns == 1 ? pages > solo : pps > kShortSplitPages) return false;
   // Open-ended, the last split holds what a sequence longer than expected has left.
-  if (cut->open_end && kernel_pages - (long long)(ns - 1) * pps > sqa::kMaxSplitPages)
+  if (kernel_pages - (long long)(ns - 1) * pps > sqa::kMaxSplitPages)
     return false;
   cut->num_splits = ns;
   cut->pages_per_split = pps;
   return true;
 }
 
-// What a call runs. A plan says which pages of every sequence are read (a fixed
-// one the first num_splits * pages_per_split, a balanced one all); how they are
-// cut changes only the order of the sums. A balanced plan of at least a wave of
-// items over short sequences takes short_cut(). A fixed plan of a caller's chunk
-// size (the reference's default is 512 keys) leaves most of the chip idle for a
-// few sequences (one of 8K keys: 32 workgroups on 256 CUs) and runs a second,
-// partly filled wave of workgroups for many: the same pages are cut as the
-// automatic plan (and short_cut) would, where the caller's workspace holds that.
-// Measured with 512-key chunks, as given -> re-cut (us per call, back to back):
-// one sequence of 8K keys 35.2 -> 13.7 (q_len 2), of 32K keys 46.1 -> 28.4; two
-// of 8K keys, q_len 8, 43.6 -> 23.9. Kept as given: plans past kMaxBalancedBatch
-// sequences (the automatic plan is then another fixed one); one split per sequence
-// (no partials, no merge) under kMinRecutPages, or where the cut would be a
-// balanced one; and, where it would be, chunks that come to between half a wave and
-// two or three waves of work items (an eighth past 32 rows, whose partial rows cost
-// most, or with many sequences): there balanced items that span sequence ends lose
-// more than idle or late workgroups do (937 shapes; 64 ragged sequences of up to 1K
-// keys, q_len 16, 2 splits each: 43 us as given, 76 balanced), while past two waves
-// the start-ups cost 7-40%.
-constexpr long long kMinRecutPages = 16;
+// What a call runs: its plan as given, or, for a balanced plan of at least a wave of
+// items over short sequences, the fixed cut of short_cut(). How a balanced plan's
+// pages are cut changes only the order of the sums; a fixed plan runs as given: a
+// chunk size cuts a sequence at the same keys whatever the batch, the table's width
+// and the chip.
 Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_pages) {
-  const Cut as_given{a.num_splits, a.pages_per_split, kernel_pages, false};
-  const bool balanced = sqa::is_balanced(a.pages_per_split);
-  if (a.batch > sqa::kMaxBalancedBatch || !a.workspace || (uintptr_t)a.workspace % 16 ||
+  const Cut as_given{a.num_splits, a.pages_per_split, false};
+  if (!sqa::is_balanced(a.pages_per_split) || a.batch < 2 || a.batch > sqa::kMaxBalancedBatch ||
       (a.flags & SQA_FLAG_ADAPTIVE_PAIRS))
     return as_given;
   int device = -1;
@@ -187,34 +167,13 @@ Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_p
   const int cus = sqa_device_cu_count(device);
   if (cus <= 0) return as_given;
   const long long wave = wave_items(cus, rows, a.num_kv_heads, a.head_dim);
+  if (a.num_splits - a.batch < wave) return as_given;
   Cut cut = as_given;
-  if (balanced) {
-    if (a.batch < 2 || a.num_splits - a.batch < wave) return as_given;
-    const int expected = sqa::spec_pages_of(a.pages_per_split);
-    cut.open_end = true;
-    if (!short_cut(wave, a.batch, rows, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
-                   kernel_pages, &cut))
-      return as_given;
-  } else {
-    cut.pages = std::min((long long)a.num_splits * a.pages_per_split, kernel_pages);
-    if (cut.pages >= (1LL << 24) || a.batch * cut.pages >= (1LL << 30) ||
-        automatic_plan(device, a.batch, rows, a.num_kv_heads, a.head_dim, cut.pages,
-                       (int)cut.pages, true, &cut.num_splits, &cut.pages_per_split) != SQA_OK)
-      return as_given;
-    const bool shorter =
-        short_cut(wave, a.batch, rows, a.num_kv_heads, cut.pages, cut.pages, &cut);
-    const long long given = (long long)a.batch * a.num_splits;
-    bool better;
-    if (a.num_splits == 1)
-      better = (shorter || a.batch == 1) && cut.pages >= kMinRecutPages;
-    else if (a.batch == 1 || shorter)
-      better = true;
-    else if (given < wave)
-      better = rows > 32 ? 8 * given <= wave : 2 * given <= wave && 8 * a.batch <= wave;
-    else
-      better = given >= 3 * wave || (given >= 2 * wave && 4 * a.batch <= wave);
-    if (!better) return as_given;
-  }
+  cut.open_end = true;
+  const int expected = sqa::spec_pages_of(a.pages_per_split);
+  if (!short_cut(wave, a.batch, rows, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
+                 kernel_pages, &cut))
+    return as_given;
   const unsigned long long part_o_bytes =
       (unsigned long long)sqa::plan_slots(a.batch, cut.num_splits, cut.pages_per_split) *
       a.num_kv_heads * rows * a.head_dim * sizeof(float);
@@ -458,7 +417,7 @@ int run_attention(const sqa_attention_args& a) {
   pa.head_dim = head_dim;
   pa.bt_stride = max_pages;
   pa.page_shift = page_shift;
-  pa.max_pages = (int)cut.pages;
+  pa.max_pages = (int)kernel_pages;
   pa.open_end = cut.open_end;
   pa.pages_per_split = balanced ? 0 : pages_per_split;
   pa.num_splits = num_splits;
@@ -542,7 +501,7 @@ int run_attention(const sqa_attention_args& a) {
     ma.group = group;
     ma.rows = (int)rows;
     ma.head_dim = head_dim;
-    ma.max_pages = (int)cut.pages;
+    ma.max_pages = (int)kernel_pages;
     ma.pages_per_split = pa.pages_per_split;
     ma.num_splits = num_splits;
     ma.spec_pages = spec_pages;
@@ -690,7 +649,7 @@ int sqa_paged_mtp_attention_noalloc(const void* query, const void* key_cache,
                                   batch, q_len, num_query_heads, num_kv_heads, head_dim, num_pages,
                                   page_size, max_pages, num_splits, pages_per_split, stream);
   a.workspace = ws;
-  a.workspace_bytes = need;  // what the plan needs: cut as a caller's workspace of that size is
+  a.workspace_bytes = need;
   return run_attention(a);
 }
 

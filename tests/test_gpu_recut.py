@@ -1,7 +1,6 @@
-"""Calls with a chunk size run the automatic cut of the same pages where their
-workspace holds it: against the float64 oracle, and against the plan run as given
-(a workspace of that plan's own size, or none), at lengths where the two differ in
-splits, items and pieces."""
+"""How calls cut their pages: a fixed plan (a chunk size) as given, whatever surrounds
+a sequence, and a balanced plan over short sequences at their starts. Against the
+float64 oracle at lengths where the two differ in splits, items and pieces."""
 
 import sys
 
@@ -35,45 +34,63 @@ def _call(tensors, ns, pps, nbytes):
 @pytest.mark.parametrize("chunk", [16, 48, 512, 1 << 20])
 @pytest.mark.parametrize("lens", [
     [1], [63], [193], [4099],                      # one sequence: 1 page .. 257 pages
-    [0, 5, 511, 513, 2050], [640] * 3, [300] * 130,  # balanced cuts, ragged, uniform, many
+    [0, 5, 511, 513, 2050], [640] * 3, [300] * 130,  # ragged, uniform, many
 ])
-def test_chunked_plans_are_cut_like_the_automatic_one(q_len, chunk, lens):
+def test_chunked_plans_run_as_given(q_len, chunk, lens):
+    """Against the oracle, and the same bits whatever the size of the workspace: the
+    splits are the plan's, where one as large as the automatic plan's is given too."""
     case = inputs.Case(batch=len(lens), q_len=q_len, seq_lens=lens, seed=2100 + q_len)
     host = inputs.make_inputs(case)
     tensors = tuple(t.cuda() for t in host)
-    q, k, v, bt, sl = tensors
+    bt = tensors[3]
     ref = attention_c64(*host, 16, 8)
     label = f"q{q_len} ck{chunk} B{len(lens)}"
-    assert_parity(sqa.paged_mtp_attention(*tensors, 16, max(lens), chunk_keys=chunk), ref,
-                  label=label)
+    out = sqa.paged_mtp_attention(*tensors, 16, max(lens), chunk_keys=chunk)
+    assert_parity(out, ref, label=label)
     b = len(lens)
     ns, pps = _lib.plan_splits(0, b, q_len, 32, 8, 128, max(lens), bt.shape[1], chunk)
     own = _lib.workspace_bytes(b, q_len, 32, 8, 128, ns, pps)
-    more = _lib.call_workspace_bytes(0, b, q_len, 32, 8, 128, ns, pps, bt.shape[1])
-    assert more >= own
-    for nbytes in {own, more}:
-        assert_parity(_call(tensors, ns, pps, nbytes), ref, label=f"{label} {nbytes} bytes")
+    for nbytes in (own, own + (64 << 20)):
+        assert torch.equal(_call(tensors, ns, pps, nbytes), out), f"{label} {nbytes} bytes"
 
 
-@pytest.mark.parametrize("batch", [1, 3])
-@pytest.mark.parametrize("splits,pps", [(1, 20), (5, 4), (40, 1)])
-def test_a_recut_plan_reads_the_pages_of_the_plan_as_given(batch, splits, pps):
-    """A plan covers the first num_splits * pages_per_split pages of every sequence
-    and no more, however it is cut: longer sequences see only those keys."""
-    lens = [1000] * batch
+@pytest.mark.parametrize("q_len", [2, 4, 8])
+@pytest.mark.parametrize("chunk", [48, 512, 1 << 20])
+def test_chunked_sequences_do_not_depend_on_their_surroundings(q_len, chunk):
+    """A chunk size cuts a sequence at the same keys alone and in a batch, under a table
+    of its own width and a wider one, promised its length and the batch's longest: the
+    same bits (the batch's rows stay within one form of the merge kernel)."""
+    lens = [700, 65, 4099] if q_len == 2 else [700, 1300]
+    q, k, v, bt, sl = (t.cuda() for t in inputs.make_inputs(
+        inputs.Case(batch=len(lens), q_len=q_len, seq_lens=lens, seed=2200 + q_len)))
+    wide = torch.zeros(len(lens), 600, dtype=torch.int32, device="cuda")
+    wide[:, :bt.shape[1]] = bt
+    together = sqa.forward_v3(q, k, v, wide, sl, 16, chunk, max(lens))
+    for i, n in enumerate(lens):
+        one = slice(i, i + 1)
+        for table in (bt[one, :-(-n // 16)].contiguous(), wide[one].contiguous()):
+            alone = sqa.forward_v3(q[one].contiguous(), k, v, table, sl[one].contiguous(), 16,
+                                   chunk, n)
+            assert torch.equal(alone, together[one]), f"{n} keys, table of {table.shape[1]}"
+
+
+@pytest.mark.parametrize("lens", [[1000], [1000] * 3, [1000, 100, 700, 330, 1], [650] * 2])
+@pytest.mark.parametrize("splits,pps", [(1, 20), (5, 4), (40, 1), (2, 20)])
+def test_a_plan_reads_its_pages_of_longer_sequences(lens, splits, pps):
+    """A plan covers the first num_splits * pages_per_split pages of every sequence and
+    no more: longer sequences see only those keys, shorter ones all of theirs."""
+    batch = len(lens)
     q, k, v, bt, sl = (t.cuda() for t in inputs.make_inputs(
         inputs.Case(batch=batch, q_len=4, seq_lens=lens, seed=2200)))
-    pages = splits * pps
     own = _lib.workspace_bytes(batch, 4, 32, 8, 128, splits, pps)
-    as_given = _call((q, k, v, bt, sl), splits, pps, own)
-    recut = _call((q, k, v, bt, sl), splits, pps, 64 << 20)
-    # The draft lies behind them: every row sees all of their keys, as a lone
-    # query at the end of a sequence of that length would.
-    short = torch.full((batch,), pages * 16, dtype=torch.int32)
-    want = attention_c64(q.cpu()[:, :1].contiguous(), k.cpu(), v.cpu(), bt.cpu(), short, 16, 8)
-    for out, label in ((as_given, "as given"), (recut, "re-cut")):
-        assert_parity(out[:, :1].contiguous(), want, label=label)
-    assert (as_given.float() - recut.float()).abs().max().item() <= 2e-3
+    out = _call((q, k, v, bt, sl), splits, pps, own)
+    # Behind them lies the draft of the longer ones: every row sees all of the keys, as a
+    # lone query at the end of a sequence of that length would.
+    cover = splits * pps * 16
+    seen = torch.tensor([min(n, cover) for n in lens], dtype=torch.int32)
+    want = attention_c64(q.cpu()[:, 3:].contiguous(), k.cpu(), v.cpu(), bt.cpu(), seen, 16, 8)
+    assert_parity(out[:, 3:].contiguous(), want, label=f"B{batch} {splits}x{pps}")
+    assert torch.equal(out, _call((q, k, v, bt, sl), splits, pps, own + (64 << 20)))
 
 
 @pytest.mark.parametrize("q_len", [2, 8, 16])
