@@ -1306,12 +1306,15 @@ __device__ __forceinline__ void wait_vmcnt_fence() {
 // One load per lane straight into LDS (gfx950 global_load_lds_*): lane l's 16 (or
 // 4) bytes land at LDS byte address lds + 16 l (4 l). Inline asm for the reason
 // given at load_to_lds: the compiler's wait-count pass must not drain the page
-// ring for it. The callers wait themselves (wait_vmcnt_fence).
+// ring for it. The callers wait themselves (wait_vmcnt_fence). The s_nop is the wait
+// state the hardware asks for between a scalar write of m0 and a load into LDS, which
+// the compiler's hazard pass does not put into inline asm.
 __device__ __forceinline__ void copy16_to_lds(const void* src, unsigned lds) {
   unsigned saved;
   asm volatile(
       "s_mov_b32 %[saved], m0\n\t"
       "s_mov_b32 m0, %[lds]\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %[src], off\n\t"
       "s_mov_b32 m0, %[saved]"
       : [saved] "=&s"(saved)
@@ -1323,6 +1326,7 @@ __device__ __forceinline__ void copy4_to_lds(const void* src, unsigned lds) {
   asm volatile(
       "s_mov_b32 %[saved], m0\n\t"
       "s_mov_b32 m0, %[lds]\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dword %[src], off\n\t"
       "s_mov_b32 m0, %[saved]"
       : [saved] "=&s"(saved)
@@ -1830,13 +1834,15 @@ __device__ __forceinline__ void wait_vmcnt() {
 // later LDS read that might alias it, which would drain a ring of these loads at
 // each step; the callers place their vmcnt waits themselves and issue no other
 // vector-memory loads meanwhile. m0 (the LDS base of the load) is saved and
-// restored around it.
+// restored around it, with the wait state (s_nop) that a load into LDS needs after a
+// write of m0.
 __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned voffset,
                                             unsigned lds) {
   unsigned saved;
   asm volatile(
       "s_mov_b32 %[saved], m0\n\t"
       "s_mov_b32 m0, %[lds]\n\t"
+      "s_nop 0\n\t"
       "buffer_load_dwordx4 %[off], %[rsrc], 0 offen nt lds\n\t"
       "s_mov_b32 m0, %[saved]"
       : [saved] "=&s"(saved)

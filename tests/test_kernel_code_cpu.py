@@ -1,0 +1,84 @@
+"""What the kernels' inline assembly relies on and the compiler does not check, read
+from the machine code of the library as it is built (llvm-objdump; no GPU)."""
+
+import functools
+import re
+import shutil
+import subprocess
+import tempfile
+from pathlib import Path
+
+import pytest
+
+from small_q_attention_amd import build as sqa_build
+
+OBJDUMP = Path("/opt/rocm/lib/llvm/bin/llvm-objdump")
+_LINE = re.compile(r"^\t(\S+)\s*(.*?)\s*// 0*([0-9A-F]+):.*?(?:<.*\+0x([0-9a-f]+)>)?$")
+
+
+@functools.lru_cache(maxsize=1)
+def kernels():
+    """``{symbol: [(address, mnemonic, operands, branch target or None)]}`` of the library."""
+    if not OBJDUMP.exists():
+        pytest.skip("no llvm-objdump")
+    if sqa_build.is_stale():
+        sqa_build.build()
+    out = {}
+    with tempfile.TemporaryDirectory() as tmp:
+        lib = Path(tmp) / "lib.so"
+        shutil.copy(sqa_build.LIB_PATH, lib)
+        subprocess.run([OBJDUMP, "--offloading", lib.name], cwd=tmp, check=True,
+                       capture_output=True)
+        for code in sorted(Path(tmp).glob("lib.so.*amdgcn*")):
+            text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code.name], cwd=tmp,
+                                  check=True, capture_output=True, text=True).stdout
+            body = None
+            for line in text.splitlines():
+                head = re.match(r"^([0-9a-f]+) <(\S+)>:$", line)
+                if head:
+                    start, body = int(head.group(1), 16), []
+                    out[head.group(2)] = body
+                    continue
+                m = _LINE.match(line)
+                if m and body is not None:
+                    to = start + int(m.group(4), 16) if m.group(4) else None
+                    body.append((int(m.group(3), 16), m.group(1), m.group(2), to))
+    assert any("sqa_partial_kernel" in k for k in out)
+    return out
+
+
+def _loads_into_lds(op, args):
+    return op.startswith("global_load_lds") or (op.startswith("buffer_load") and
+                                                args.split()[-1] == "lds")
+
+
+def _scalars(text):
+    """Numbers of the scalar registers named in an operand list."""
+    regs = {int(n) for n in re.findall(r"\bs(\d+)\b", text)}
+    for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+        regs |= set(range(int(lo), int(hi) + 1))
+    return regs
+
+
+def test_loads_into_lds_keep_their_wait_states():
+    """A load into LDS takes its LDS address from m0 and its base from scalar registers:
+    one wait state after a scalar write of m0, five after a vector instruction's write of
+    a scalar register it reads. The compiler keeps them for its own instructions and does
+    not look into inline assembly."""
+    seen = 0
+    for name, code in kernels().items():
+        for i, (_, op, args, _) in enumerate(code):
+            if not _loads_into_lds(op, args):
+                continue
+            seen += 1
+            reads, states = _scalars(args), 0
+            for _, prev, pargs, _ in reversed(code[max(0, i - 5):i]):
+                dest = pargs.split(",")[0]
+                if prev.startswith("s_") and dest == "m0":
+                    assert states >= 1, f"{name}: {op} right after {prev} m0"
+                if prev.startswith("v_"):
+                    assert states >= 5 or not reads & _scalars(dest), f"{name}: {prev} {pargs}"
+                states += 1 + (int(pargs, 0) if prev == "s_nop" else 0)
+                if states >= 5:
+                    break
+    assert seen > 0
