@@ -56,11 +56,12 @@ extern "C" {
  *     ragged batches spread evenly over the chip without a host sync. With
  *     max_seq_len > 0 it is -P, P = ceil(max_seq_len / 16) (at most max_pages):
  *     the kernels first assume every sequence spans P pages, which saves a
- *     memory round trip when it holds, and verify it (the result is the same
- *     either way). Otherwise a fixed plan as above. A call whose sequences are
- *     short (P pages, or the whole table row, in splits of a few pages) cuts
- *     every sequence from its own start instead, as a fixed plan does, reading
- *     the same pages.
+ *     memory round trip when it holds, and verify it (the keys read are the same
+ *     either way, and so are the result's bits where items are longer than 4
+ *     pages and neither paired nor counted per head group). A call whose table
+ *     rows are short (max_pages in splits of a few pages) cuts every sequence
+ *     from its own start instead, as a fixed plan does, reading the same pages,
+ *     with and without a P. Other batches: a fixed plan as above.
  * max_pages: 16-token pages a block-table row addresses (block_tables columns
  * x page_size / 16); num_splits and pages_per_split count 16-token pages too.
  * max_seq_len <= 0 means "unknown": a fixed plan covers max_pages * 16 tokens.

@@ -106,12 +106,6 @@ int automatic_plan(int device, int batch, long long rows, int num_kv_heads, int 
   return fixed_plan(batch, num_kv_heads, pages, pps, num_splits, pages_per_split);
 }
 
-// How a call cuts the pages of its plan.
-struct Cut {
-  int num_splits, pages_per_split;
-  bool open_end;  // fixed: the last split of a sequence runs to its end
-};
-
 // Short sequences: a balanced item of a few pages spans sequence ends, and every
 // piece of it and every merged row costs as much as the pages. So where each
 // sequence's own share of the wave's items, `per_seq`, cuts its pages into splits
@@ -130,58 +124,43 @@ struct Cut {
 // whose partial rows cost most (64 of 32 pages, q_len 16: 1.3x).
 constexpr long long kShortSplitPages = 12, kSoloPages = 8, kShortSinglePages = 32;
 bool short_cut(long long items, int batch, long long rows, int num_kv_heads, long long pages,
-               long long kernel_pages, Cut* cut) {
+               int* num_splits, int* pages_per_split) {
   const long long per_seq = std::max(1LL, items / batch);
   const long long solo = per_seq == 1 || (per_seq == 2 && rows > 32) ? kShortSinglePages
                          : rows <= 32 || per_seq <= 4                ? kSoloPages
                                                                      : sqa::kMinSplitPages;
-  // Splits of an even number of pages: lengths expected a page or two apart (a
-  // caller's longest length and its table's width) mostly get the same cut, so the
-  // same bits.
+  // An even number of pages per split, as in the shapes measured.
   long long want = std::max(ceil_div(pages, per_seq), (long long)sqa::kMinSplitPages);
   want += want & 1;
   if (pages <= solo) want = pages;
   int ns = 0, pps = 0;
   if (fixed_plan(batch, num_kv_heads, pages, want, &ns, &pps) != SQA_OK) return false;
   if (ns == 1 ? pages > solo : pps > kShortSplitPages) return false;
-  // Open-ended, the last split holds what a sequence longer than expected has left.
-  if (kernel_pages - (long long)(ns - 1) * pps > sqa::kMaxSplitPages)
-    return false;
-  cut->num_splits = ns;
-  cut->pages_per_split = pps;
+  *num_splits = ns;
+  *pages_per_split = pps;
   return true;
 }
 
-// What a call runs: its plan as given, or, for a balanced plan of at least a wave of
-// items over short sequences, the fixed cut of short_cut(). How a balanced plan's
-// pages are cut changes only the order of the sums; a fixed plan runs as given: a
-// chunk size cuts a sequence at the same keys whatever the batch, the table's width
-// and the chip.
-Cut cut_for_call(const sqa_attention_args& a, long long rows, long long kernel_pages) {
-  const Cut as_given{a.num_splits, a.pages_per_split, false};
+// Replaces a balanced plan of at least a wave of items by the fixed cut of
+// short_cut() where the block table's rows are short enough: how a balanced plan's
+// pages are cut changes only the order of the sums. The rule looks at the table's
+// width and not at the pages a caller expects (pages_per_split -P), which must not
+// change the result's bits. A fixed plan runs as given: a chunk size cuts a sequence
+// at the same keys whatever the batch, the table's width and the chip.
+// The cut has at most per_seq splits per sequence, so fewer partial slots than the
+// plan it replaces: that plan's workspace and limits hold it.
+void cut_short_sequences(const sqa_attention_args& a, long long rows, long long kernel_pages,
+                         int* num_splits, int* pages_per_split) {
   if (!sqa::is_balanced(a.pages_per_split) || a.batch < 2 || a.batch > sqa::kMaxBalancedBatch ||
       (a.flags & SQA_FLAG_ADAPTIVE_PAIRS))
-    return as_given;
+    return;
   int device = -1;
-  if (hipGetDevice(&device) != hipSuccess) return as_given;
+  if (hipGetDevice(&device) != hipSuccess) return;
   const int cus = sqa_device_cu_count(device);
-  if (cus <= 0) return as_given;
+  if (cus <= 0) return;
   const long long wave = wave_items(cus, rows, a.num_kv_heads, a.head_dim);
-  if (a.num_splits - a.batch < wave) return as_given;
-  Cut cut = as_given;
-  cut.open_end = true;
-  const int expected = sqa::spec_pages_of(a.pages_per_split);
-  if (!short_cut(wave, a.batch, rows, a.num_kv_heads, expected > 0 ? expected : kernel_pages,
-                 kernel_pages, &cut))
-    return as_given;
-  const unsigned long long part_o_bytes =
-      (unsigned long long)sqa::plan_slots(a.batch, cut.num_splits, cut.pages_per_split) *
-      a.num_kv_heads * rows * a.head_dim * sizeof(float);
-  if (part_o_bytes > sqa::kMaxPartialBytes ||
-      sqa_workspace_bytes(a.batch, a.q_len, a.num_query_heads, a.num_kv_heads, a.head_dim,
-                          cut.num_splits, cut.pages_per_split) > a.workspace_bytes)
-    return as_given;
-  return cut;
+  if (a.num_splits - a.batch >= wave)
+    short_cut(wave, a.batch, rows, a.num_kv_heads, kernel_pages, num_splits, pages_per_split);
 }
 
 }  // namespace
@@ -377,9 +356,7 @@ int run_attention(const sqa_attention_args& a) {
   if ((balanced || num_splits > 1) && part_o_bytes > sqa::kMaxPartialBytes)
     return fail(SQA_ERR_INVALID, "the plan's partials (%llu bytes) exceed %llu bytes",
                 part_o_bytes, sqa::kMaxPartialBytes);
-  const Cut cut = cut_for_call(a, rows, kernel_pages);
-  num_splits = cut.num_splits;
-  pages_per_split = cut.pages_per_split;
+  cut_short_sequences(a, rows, kernel_pages, &num_splits, &pages_per_split);
   balanced = sqa::is_balanced(pages_per_split);
   spec_pages = sqa::spec_pages_of(pages_per_split);
   part_o_bytes = partial_bytes();
@@ -418,7 +395,6 @@ int run_attention(const sqa_attention_args& a) {
   pa.bt_stride = max_pages;
   pa.page_shift = page_shift;
   pa.max_pages = (int)kernel_pages;
-  pa.open_end = cut.open_end;
   pa.pages_per_split = balanced ? 0 : pages_per_split;
   pa.num_splits = num_splits;
   pa.spec_pages = spec_pages;

@@ -168,7 +168,6 @@ struct PartialArgs {
   int page_shift;             // cache page = 16 << page_shift tokens = 1 << page_shift kernel pages
   int max_pages;              // kernel pages a block-table row addresses (bt_stride << page_shift)
   int pages_per_split, num_splits;
-  int open_end;               // fixed plan: a sequence's last split runs to its end
   int spec_pages;             // balanced plan: expected pages of every sequence (0: none)
   int spec_pps;               // the balanced plan's item size when every sequence spans spec_pages
   int seam_pages;             // balanced plan: pages a second piece costs a workgroup (0: no gaps)

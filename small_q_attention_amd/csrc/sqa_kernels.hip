@@ -738,8 +738,7 @@ __device__ __forceinline__ ItemRange fixed_item(const PartialArgs& a, int item) 
   r.p_begin = r.split * a.pages_per_split;
   r.len = max(scalar_load(a.seq_lens + r.b), 0);
   const int pages = min((r.len + kPageSize - 1) / kPageSize, a.max_pages);
-  const bool rest = a.open_end && r.split == a.num_splits - 1;
-  r.p_end = rest ? pages : min(r.p_begin + a.pages_per_split, pages);
+  r.p_end = min(r.p_begin + a.pages_per_split, pages);
   r.n_valid = min(pages > a.pages_per_split ? 2 : (int)(pages > 0), a.num_splits);
   r.slot0 = r.b * a.num_splits;
   r.g_end = 0;
@@ -1408,7 +1407,7 @@ void sqa_partial_kernel(PartialArgs a) {
                "s"(a.num_splits), "s"(a.pages_per_split), "s"(a.bt_stride), "s"(a.max_pages),
                "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.hg_items[0]),
                "s"(a.by_head_groups.mul), "s"(a.by_head_groups.shift), "s"(a.by_splits.mul),
-               "s"(a.by_splits.shift), "s"(a.open_end));
+               "s"(a.by_splits.shift));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // blockIdx.x = item * head_groups + head_group, or with items per head group
@@ -1913,7 +1912,7 @@ void sqa_partial_lds_kernel(PartialArgs a) {
                "s"(a.num_splits), "s"(a.pages_per_split), "s"(a.bt_stride), "s"(a.max_pages),
                "s"(a.page_shift), "s"(a.spec_pages), "s"(a.spec_pps), "s"(a.pair_items),
                "s"(a.by_head_groups.mul), "s"(a.by_head_groups.shift), "s"(a.by_splits.mul),
-               "s"(a.by_splits.shift), "s"(a.open_end));
+               "s"(a.by_splits.shift));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // blockIdx.x = item * head_groups + head_group; with paired items (two head

@@ -114,3 +114,27 @@ def test_short_sequences_are_cut_at_their_starts(q_len, lens, promise, width):
         out = sqa.paged_mtp_attention(*dev, 16, given)
         assert_parity(out, ref, label=f"q{q_len} B{len(lens)} promise {given}")
         assert torch.equal(out, sqa.paged_mtp_attention(*dev, 16, given))
+
+
+@pytest.mark.parametrize("q_len", [2, 8])
+@pytest.mark.parametrize("lens,width", [
+    ([1500] * 8, 200),                                 # too wide a table for the cut
+    ([1500, 90, 700, 1499, 0, 33, 1200, 1500], 200),
+    ([700] * 5, 300), ([1100] * 5, 300),               # splits of 12 pages
+    ([100] * 64, 7), ([100] * 64, 9), ([400] * 40, 60),
+])
+def test_a_promised_length_does_not_change_the_bits(q_len, lens, width):
+    """The cut of short sequences looks at the table's width, the same whatever length is
+    promised, and at no more of the workspace than the plan asks for."""
+    case = inputs.Case(batch=len(lens), q_len=q_len, seq_lens=lens, seed=2600 + q_len)
+    q, k, v, bt, sl = inputs.make_inputs(case)
+    wide = torch.zeros(len(lens), width, dtype=torch.int32)
+    wide[:, :bt.shape[1]] = bt
+    dev = tuple(t.cuda() for t in (q, k, v, wide, sl))
+    plain = sqa.paged_mtp_attention(*dev, 16, 0)
+    assert_parity(plain, attention_c64(q, k, v, bt, sl, 16, 8), label=f"q{q_len} width {width}")
+    for promise in (max(lens), max(lens) + 16, (max(lens) + width * 16) // 2, width * 16):
+        assert torch.equal(sqa.paged_mtp_attention(*dev, 16, promise), plain), promise
+        ns, pps = _lib.plan_splits(0, len(lens), q_len, 32, 8, 128, promise, width, 0)
+        own = _lib.workspace_bytes(len(lens), q_len, 32, 8, 128, ns, pps)
+        assert torch.equal(_call(dev, ns, pps, own + (64 << 20)), plain), promise
