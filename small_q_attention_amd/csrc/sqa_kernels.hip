@@ -595,6 +595,15 @@ __device__ __forceinline__ void page_finish(WaveState<NB, HD>& st, f4 (&s)[NB],
   page_pv<NB, HD, E, KV, HPW>(st, s, pv, upper, c);
 }
 
+// threadIdx.x through an empty asm statement: what a piece of work, or a rare branch
+// of one, derives from it is computed there, not hoisted by the compiler in front of
+// the loop over pieces, where it would hold registers through every page loop.
+__device__ __forceinline__ int piece_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Two pages in one softmax step: fp16 queries over an e4m3 cache at head dim
 // 128, one kv head per wave (the 64-row kernel, where the math, not the bytes,
 // sets the time). s0 / s1: the raw scores of pages p and p + 1; r0 / r1 their
@@ -611,7 +620,7 @@ template <int NB, typename Bits>
 __device__ __forceinline__ void pair_finish(WaveState<NB, 128>& st, f4 (&s0)[NB], f4 (&s1)[NB],
                                             KvFp8<128>::Regs r0, KvFp8<128>::Regs r1,
                                             bool have1, const Bits& bits, int draft_base,
-                                            int tok0, int len, bool masked, float c) {
+                                            int tok_base, int len, bool masked, float c) {
   using E = ElemF16;
   constexpr int MB = Dims<128>::MB;
   // Both conditions are uniform over the wave and rare (pages at the draft
@@ -621,6 +630,7 @@ __device__ __forceinline__ void pair_finish(WaveState<NB, 128>& st, f4 (&s0)[NB]
     if (masked) {
       unsigned long long dbits[NB];
       bits.get(dbits);
+      const int tok0 = tok_base + 4 * ((piece_tid() & 63) >> 4);
       mask_scores<NB>(s0, dbits, draft_base, tok0, len);
       mask_scores<NB>(s1, dbits, draft_base, tok0 + kPageSize, len);
 #pragma unroll
@@ -744,15 +754,6 @@ __device__ __forceinline__ ItemRange fixed_item(const PartialArgs& a, int item) 
   r.g_end = 0;
   r.paired = 0;
   return r;
-}
-
-// threadIdx.x through an empty asm statement: what a piece of work derives from
-// it is computed inside that piece, not hoisted by the compiler in front of the
-// loop over pieces, where it would hold registers through every page loop.
-__device__ __forceinline__ int piece_tid() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
 }
 
 // Inclusive prefix sum over the wave's 64 lanes with DPP: within rows of 16
@@ -1345,16 +1346,21 @@ struct RegBits {
 
 // Draft bits of a wave's rows: the caller's mask words, copied to LDS with the
 // piece's Q (block nb's row r: word w at 32 nb + 16 w + r), or the causal chain.
-// Padding rows get some row's bits; they are never stored.
-template <int NB, int HPW>
+// Padding rows get some row's bits; they are never stored. FIND: get() finds the
+// lane for itself. The e4m3 64-row kernel needs that: held through its page loop, the
+// lane and what follows from it took a pair of ring registers, whose copies waited for
+// a load just issued (16 x 32K keys, q_len 16, per call: 212.8 against 193.0 us). At 32 rows the branch
+// around it costs the pipelined loop its overlap (e4m3 q_len 8 172.4 -> 195.3 us).
+template <int NB, int HPW, bool FIND>
 struct StagedBits {
   const unsigned* words;
   bool masked;            // the caller's words; else the causal chain
   bool two;               // two words per row
   FastDiv by_group;
-  int l16;
+  int lane16;
   WaveRows<NB, HPW> map;
   __device__ __forceinline__ void get(unsigned long long (&dbits)[NB]) const {
+    const int l16 = FIND ? piece_tid() & 15 : lane16;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       if (masked) {  // uniform
@@ -1606,8 +1612,8 @@ void sqa_partial_kernel(PartialArgs a) {
   // This piece's Q and mask words are in LDS: D pages were requested after them.
   wait_vmcnt_fence<D * HPW * KV::kLoads>();
   const u4* q_lds = my_q + (buf % kQBufs) * kQLds;
-  const StagedBits<NB, HPW> bits{my_bits + buf * kBitsLds, a.draft_mask != nullptr,
-                                 a.mask_words > 1, a.by_group, l16, map};
+  const StagedBits<NB, HPW, kPairSteps> bits{my_bits + buf * kBitsLds, a.draft_mask != nullptr,
+                                             a.mask_words > 1, a.by_group, l16, map};
   // Pages holding a token >= mask_from (draft block or past the end) are masked.
   const int mask_from = len - a.q_len;
 
@@ -1695,7 +1701,7 @@ void sqa_partial_kernel(PartialArgs a) {
             }
           }
           pair_finish<NB>(st, s0, s1, ring[j][0], ring[j + 1][0], ii + 1 < n_pages, bits,
-                          mask_from, p * kPageSize + 4 * g16, len, masked, a.scale_log2);
+                          mask_from, p * kPageSize, len, masked, a.scale_log2);
         }
         const int pid0 = next_pid;
         const int pid1 = page_id(f + ii + D + 1);

@@ -82,3 +82,40 @@ def test_loads_into_lds_keep_their_wait_states():
                 if states >= 5:
                     break
     assert seen > 0
+
+
+_LOADS = {("KvNative", 64): 6, ("KvNative", 128): 8, ("KvNative", 256): 16,
+          ("KvFp8", 64): 5, ("KvFp8", 128): 6, ("KvFp8", 256): 8}  # per page and head
+
+
+def _partial_kernels():
+    """``(symbol, code, pages of the ring, load instructions per page of a wave)``."""
+    for name, code in kernels().items():
+        m = re.search(r"sqa_partial_kernelILi\d+ELi(\d+)ELi\d+ELi\d+ELi(\d+)ENS0_\d+Elem\w+?"
+                      r"ENS0_\d+(Kv[A-Za-z0-9]+?)ILi\d+EEELi(\d)E", name)
+        if m:
+            pages, hd, kv, heads = int(m.group(1)), int(m.group(2)), m.group(3), int(m.group(4))
+            yield name, code, pages, _LOADS[kv, hd] * heads
+
+
+def test_the_page_loop_never_drains_its_ring():
+    """In a turn of the page loop the wave waits for the pages it is about to use, with
+    the others in flight. A ring register moved elsewhere at the turn's end waits for a
+    load just issued instead."""
+    for name, code, pages, loads in _partial_kernels():
+        at = {ins[0]: i for i, ins in enumerate(code)}
+        turns = []
+        for i, (addr, _, _, to) in enumerate(code):
+            if to is not None and to <= addr and to in at:
+                body = code[at[to]:i + 1]
+                n = sum(op.startswith("buffer_load") for _, op, _, _ in body)
+                if n == pages * loads and not any(op.startswith("global_store")
+                                                  for _, op, _, _ in body):
+                    turns.append(body)
+        assert turns, name
+        waits = [int(w) for _, op, args, _ in min(turns, key=len) if op == "s_waitcnt"
+                 for w in re.findall(r"vmcnt\((\d+)\)", args)]
+        # One page is used per step, two where the step takes a pair of pages or
+        # computes the next page's scores ahead.
+        least = (pages - (2 if pages > 2 else 1)) * loads
+        assert waits and min(waits) >= least, f"{name}: waits {waits}, {least} loads in flight"
