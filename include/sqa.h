@@ -57,8 +57,8 @@ extern "C" {
  *     max_seq_len > 0 it is -P, P = ceil(max_seq_len / 16) (at most max_pages):
  *     the kernels first assume every sequence spans P pages, which saves a
  *     memory round trip when it holds, and verify it (the keys read are the same
- *     either way, and so are the result's bits where items are longer than 4
- *     pages and neither paired nor counted per head group). A call whose table
+ *     either way, and so are the result's bits where items are neither paired
+ *     nor counted per head group). A call whose table
  *     rows are short (max_pages in splits of a few pages) cuts every sequence
  *     from its own start instead, as a fixed plan does, reading the same pages,
  *     with and without a P. Other batches: a fixed plan as above.

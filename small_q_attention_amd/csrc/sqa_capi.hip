@@ -443,12 +443,10 @@ int run_attention(const sqa_attention_args& a) {
       pa.spec_pps = pps0;
     }
   }
-  // Pieces that fit the register ring take it in one softmax step: fixed plans
-  // of at most kRingPages pages per split, balanced plans whose expected items
-  // are that short (pieces can only be shorter than their item).
-  pa.ring_batch = head_dim == 128 && kv_bytes == 2 && rows <= 32 &&
-                  (balanced ? (spec_pages > 0 && pa.spec_pps <= sqa::kRingPages)
-                            : pages_per_split <= sqa::kRingPages);
+  // Splits that fit the register ring take it in one softmax step: fixed plans of at
+  // most kRingPages pages per split.
+  pa.ring_batch = !balanced && pages_per_split <= sqa::kRingPages && head_dim == 128 &&
+                  kv_bytes == 2 && rows <= 32;
   pa.scale_log2 = (float)(1.4426950408889634 * (double)a.scale);
   pa.out_scale = a.out_scale;
   pa.bf16 = a.dtype == SQA_DTYPE_BF16;

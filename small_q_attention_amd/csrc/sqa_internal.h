@@ -172,7 +172,7 @@ struct PartialArgs {
   int spec_pps;               // the balanced plan's item size when every sequence spans spec_pages
   int seam_pages;             // balanced plan: pages a second piece costs a workgroup (0: no gaps)
   int pair_items;             // kPairsOff, kPairsAdaptive or kPairsFixed (see above)
-  int ring_batch;             // every piece expected within the register ring (kRingPages)
+  int ring_batch;             // fixed plan: every split within the register ring (kRingPages)
   int hg_items[2];            // items per head group (HeadGroupItems below); 0: both
                               // num_splits - batch, the usual layout
   int hg_spec_pps1;           // with hg_items: head group 1's item size (spec_pps: group 0's)
@@ -271,8 +271,8 @@ inline LaunchShape launch_shape(int rows, int hkv, int head_dim) {
 }
 
 // Pages the register ring of the one-wave-per-head kernel holds at head dim 128
-// with 16-bit K/V and up to 32 rows: pieces of at most this many pages take the
-// whole-ring softmax step (PartialArgs::ring_batch).
+// with 16-bit K/V and up to 32 rows: a fixed plan's splits of at most this many pages
+// take the whole-ring softmax step (PartialArgs::ring_batch).
 constexpr int kRingPages = 4;
 
 // What a second piece costs a workgroup of the balanced plan, in pages of its

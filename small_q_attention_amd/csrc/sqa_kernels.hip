@@ -1349,8 +1349,9 @@ struct RegBits {
 // Padding rows get some row's bits; they are never stored. FIND: get() finds the
 // lane for itself. The e4m3 64-row kernel needs that: held through its page loop, the
 // lane and what follows from it took a pair of ring registers, whose copies waited for
-// a load just issued (16 x 32K keys, q_len 16, per call: 212.8 against 193.0 us). At 32 rows the branch
-// around it costs the pipelined loop its overlap (e4m3 q_len 8 172.4 -> 195.3 us).
+// a load just issued (16 x 32K keys, q_len 16, per call: 212.8 against 193.0 us). At
+// 32 rows the branch around it costs the pipelined loop its overlap (e4m3 q_len 8
+// 172.4 -> 195.3 us).
 template <int NB, int HPW, bool FIND>
 struct StagedBits {
   const unsigned* words;
@@ -1442,7 +1443,8 @@ void sqa_partial_kernel(PartialArgs a) {
   constexpr bool kPipelined = NB >= 2 && D >= 3 && NB * HD <= 256;
   constexpr bool kPairSteps = __is_same(E, ElemF16) && KV::kBytes == 1 && HD == 128 &&
                               NB == 4 && HPW == 1 && D % 2 == 0;
-  constexpr bool kRingBatch = RB && KV::kBytes == 2 && HD <= 128;
+  static_assert(!RB || (!BAL && KV::kBytes == 2 && HD <= 128 && D >= kRingPages),
+                "whole-ring steps: fixed plans over 16-bit K/V");
   constexpr bool kQRegs =
       ((NB == 4 && KV::kBytes == 1) || HD == 256) && HPW == 1 && !kPipelined;
 
@@ -1652,10 +1654,13 @@ void sqa_partial_kernel(PartialArgs a) {
   // -1.5%).
   // fp16 queries over an e4m3 cache at 64 rows and head dim 128 take the
   // pages two at a time (pair_finish).
-  // A piece that fits the ring in one softmax step (below), in the RB
-  // instantiations only (the host picks them for plans whose pieces fit the
-  // ring: with the step in it, the kernel's page loop for long pieces ran 1-2%
-  // slower): 16-bit K/V, whose ring registers the MFMAs read as they are.
+  // Splits that fit the ring in one softmax step (below) in instantiations of their
+  // own, RB, for fixed plans of so few pages per split: 16-bit K/V, whose ring
+  // registers the MFMAs read as they are. Balanced items of so few pages take the
+  // loop: the step's refill of the ring for the next piece waited for its loads (4
+  // sequences of 1000 keys under a wide table, q_len 2 / 4 / 8: 14.9 / 15.0 / 18.0 us
+  // per call with the step, 13.3 / 13.6 / 15.9 without), and the bits would follow the
+  // pages a caller expects.
   int next_pid = page_id(f + D);
   if constexpr (kPairSteps) {
     // The Q fragments stay in registers for the whole loop (16 x 4 dwords; the
@@ -1710,13 +1715,13 @@ void sqa_partial_kernel(PartialArgs a) {
         load_page(pid1, p_ahead + j + 1, ring[j + 1]);
       }
     }
-  } else if (kRingBatch && n_pages <= D) {  // uniform: the whole piece is in the ring
-    // Short pieces (one sequence of 8K keys in 4-page splits, every piece of a
+  } else if constexpr (RB) {  // the whole split is in the ring
+    // Short splits (one sequence of 8K keys in 4-page splits, every split of a
     // 1K-key sequence): the ring's pages arrive together, so they are taken in
     // one softmax step, all scores first, one running-max update, then the PV
     // products, instead of D dependent page steps (the MFMAs of all pages
     // issue back to back; one sequence of 8K keys, whole calls: q_len 2 14.1
-    // -> 13.7 us, q_len 4 14.8 -> 14.2 us). Zero pages past the piece take no
+    // -> 13.7 us, q_len 4 14.8 -> 14.2 us). Zero pages past the split take no
     // part.
     f4 sb[D][NB];
     PageV<HD, HPW> pvb[D];
@@ -1746,10 +1751,6 @@ void sqa_partial_kernel(PartialArgs a) {
 #pragma unroll
     for (int j = 0; j < D; ++j)
       if (j < n_pages) page_pv<NB, HD, E, KV, HPW>(st, sb[j], pvb[j], upper, a.scale_log2);
-    if (more) {  // uniform
-#pragma unroll
-      for (int j = 0; j < D; ++j) load_page(page_id(f + D + j), next_begin + j, ring[j]);
-    }
   } else {
   f4 s_cur[NB];
   if constexpr (kPipelined)
@@ -2493,20 +2494,20 @@ void launch_partial_hd(const PartialArgs& a, const LaunchShape& sh, dim3 grid, d
                            stream, a);
     }
   } else if (sh.row_blocks == 1) {
-    if constexpr (HD == 128 && KV::kBytes == 2) {
+    if constexpr (HD == 128 && KV::kBytes == 2 && !BAL) {
       if (a.ring_batch) {
-        hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block, 0,
-                           stream, a);
+        hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block,
+                           0, stream, a);
         return;
       }
     }
     hipLaunchKernelGGL((sqa_partial_kernel<1, D4, 4, 1, HD, E, KV, 1, BAL>), grid, block, 0, stream,
                        a);
   } else if (sh.row_blocks == 2) {
-    if constexpr (HD == 128 && KV::kBytes == 2) {
+    if constexpr (HD == 128 && KV::kBytes == 2 && !BAL) {
       if (a.ring_batch) {
-        hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block, 0,
-                           stream, a);
+        hipLaunchKernelGGL((sqa_partial_kernel<2, D4, 4, 1, HD, E, KV, 1, BAL, true>), grid, block,
+                           0, stream, a);
         return;
       }
     }

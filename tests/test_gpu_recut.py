@@ -122,6 +122,7 @@ def test_short_sequences_are_cut_at_their_starts(q_len, lens, promise, width):
     ([1500, 90, 700, 1499, 0, 33, 1200, 1500], 200),
     ([700] * 5, 300), ([1100] * 5, 300),               # splits of 12 pages
     ([100] * 64, 7), ([100] * 64, 9), ([400] * 40, 60),
+    ([500] * 8, 2000), ([1000] * 4, 1500), ([16, 90, 250] * 10, 2000),  # short items
 ])
 def test_a_promised_length_does_not_change_the_bits(q_len, lens, width):
     """The cut of short sequences looks at the table's width, the same whatever length is
