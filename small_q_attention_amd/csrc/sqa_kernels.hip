@@ -1611,7 +1611,8 @@ void sqa_partial_kernel(PartialArgs a) {
   const bool more = balanced && piece_at(a, walk, item, it.g_end);
   const int next_begin = walk.it.p_begin;
   if (kQBufs == 2 && more) fetch_rows(walk.it.b, buf ^ 1);
-  // This piece's Q and mask words are in LDS: D pages were requested after them.
+  // This piece's Q and mask words are in LDS: D pages were requested after them, each
+  // in kLoads instructions per head (tests/test_kernel_code_cpu.py counts them).
   wait_vmcnt_fence<D * HPW * KV::kLoads>();
   const u4* q_lds = my_q + (buf % kQBufs) * kQLds;
   const StagedBits<NB, HPW, kPairSteps> bits{my_bits + buf * kBitsLds, a.draft_mask != nullptr,

@@ -122,3 +122,21 @@ def test_the_page_loop_never_drains_its_ring():
         # computes the next page's scores ahead.
         least = (pages - (2 if pages > 2 else 1)) * loads
         assert waits and min(waits) >= least, f"{name}: waits {waits}, {least} loads in flight"
+
+
+def test_the_wait_for_a_piece_s_rows_counts_the_loads_behind_them():
+    """A piece begins by waiting until no more vector loads are in flight than a full ring
+    has: its Q and mask words, copied into LDS before the ring's pages were requested, are
+    there then. The count is written in the source; the instructions are the compiler's."""
+    for name, code, pages, loads, _ in _partial_kernels():
+        ops = [op for _, op, _, _ in code]
+        assert ops.count("s_barrier") == 1, name
+        barrier = ops.index("s_barrier")
+        copies = [i for i, op in enumerate(ops[:barrier]) if op.startswith("global_load_lds")]
+        assert copies, name
+        behind = ops[copies[-1]:barrier]
+        assert sum(op.startswith("buffer_load") for op in behind) == pages * loads, name
+        # The six-bit counter's 63 waits for at least as much.
+        want = f"vmcnt({min(pages * loads, 63)})"
+        assert any(op == "s_waitcnt" and args.strip() == want
+                   for _, op, args, _ in code[barrier:]), f"{name}: no {want} behind the barrier"
