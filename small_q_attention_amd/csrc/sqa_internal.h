@@ -164,17 +164,19 @@ struct PartialArgs {
   int mask_words;             // 32-bit words per draft-mask row (1 or 2)
   int batch, q_len, hq, hkv, group, rows;
   int head_dim;               // 64, 128 or 256
+  // bt_stride .. hg_items[0]: eight words every kernel asks for first (with an unused
+  // one among them, its register was taken for another load and split the trip in two).
   int bt_stride;              // block_tables row length (cache pages)
   int page_shift;             // cache page = 16 << page_shift tokens = 1 << page_shift kernel pages
   int max_pages;              // kernel pages a block-table row addresses (bt_stride << page_shift)
   int pages_per_split, num_splits;
   int spec_pages;             // balanced plan: expected pages of every sequence (0: none)
   int spec_pps;               // the balanced plan's item size when every sequence spans spec_pages
+  int hg_items[2];            // items per head group (HeadGroupItems below); 0: both
+                              // num_splits - batch, the usual layout
   int seam_pages;             // balanced plan: pages a second piece costs a workgroup (0: no gaps)
   int pair_items;             // kPairsOff, kPairsAdaptive or kPairsFixed (see above)
   int ring_batch;             // fixed plan: every split within the register ring (kRingPages)
-  int hg_items[2];            // items per head group (HeadGroupItems below); 0: both
-                              // num_splits - batch, the usual layout
   int hg_spec_pps1;           // with hg_items: head group 1's item size (spec_pps: group 0's)
   float* tune;                // adaptive paired items: {magic, delta, stamp, -} then per
                               // workgroup {loop ticks, pages}

@@ -140,3 +140,16 @@ def test_the_wait_for_a_piece_s_rows_counts_the_loads_behind_them():
         want = f"vmcnt({min(pages * loads, 63)})"
         assert any(op == "s_waitcnt" and args.strip() == want
                    for _, op, args, _ in code[barrier:]), f"{name}: no {want} behind the barrier"
+
+
+def test_the_arguments_on_the_way_to_the_first_load_come_in_one_trip():
+    """The main kernel asks for the arguments it needs first at once. The order of the
+    argument record decides whether the compiler can (a register of an unused word taken
+    for a later load splits the trip in two)."""
+    for name, code, _, _, _ in _partial_kernels():
+        waits = 0
+        for _, op, args, _ in code:
+            waits += op == "s_waitcnt" and "lgkmcnt" in args
+            if op.startswith("global_load") or (op.startswith("s_load") and "s[0:1]" not in args):
+                break
+        assert waits == 1, f"{name}: {waits} trips"
