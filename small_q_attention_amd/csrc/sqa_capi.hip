@@ -150,14 +150,10 @@ bool short_cut(long long items, int batch, long long rows, int num_kv_heads, lon
 // The cut has at most per_seq splits per sequence, so fewer partial slots than the
 // plan it replaces: that plan's workspace and limits hold it.
 void cut_short_sequences(const sqa_attention_args& a, long long rows, long long kernel_pages,
-                         int* num_splits, int* pages_per_split) {
+                         int cus, int* num_splits, int* pages_per_split) {
   if (!sqa::is_balanced(a.pages_per_split) || a.batch < 2 || a.batch > sqa::kMaxBalancedBatch ||
-      (a.flags & SQA_FLAG_ADAPTIVE_PAIRS))
+      (a.flags & SQA_FLAG_ADAPTIVE_PAIRS) || cus <= 0)
     return;
-  int device = -1;
-  if (hipGetDevice(&device) != hipSuccess) return;
-  const int cus = sqa_device_cu_count(device);
-  if (cus <= 0) return;
   const long long wave = wave_items(cus, rows, a.num_kv_heads, a.head_dim);
   if (a.num_splits - a.batch >= wave)
     short_cut(wave, a.batch, rows, a.num_kv_heads, kernel_pages, num_splits, pages_per_split);
@@ -356,7 +352,11 @@ int run_attention(const sqa_attention_args& a) {
   if ((balanced || num_splits > 1) && part_o_bytes > sqa::kMaxPartialBytes)
     return fail(SQA_ERR_INVALID, "the plan's partials (%llu bytes) exceed %llu bytes",
                 part_o_bytes, sqa::kMaxPartialBytes);
-  cut_short_sequences(a, rows, kernel_pages, &num_splits, &pages_per_split);
+  int device = -1;
+  const int cus = (balanced || num_splits > 1) && hipGetDevice(&device) == hipSuccess
+                      ? sqa_device_cu_count(device)
+                      : 0;
+  cut_short_sequences(a, rows, kernel_pages, cus, &num_splits, &pages_per_split);
   balanced = sqa::is_balanced(pages_per_split);
   spec_pages = sqa::spec_pages_of(pages_per_split);
   part_o_bytes = partial_bytes();
@@ -492,7 +492,7 @@ int run_attention(const sqa_attention_args& a) {
     ma.bf16 = pa.bf16;
     ma.tune = pa.pair_items == sqa::kPairsAdaptive ? pa.tune : nullptr;
     ma.tune_records = (num_splits - batch) * 2;
-    if ((e = sqa::launch_merge(ma, s)) != hipSuccess) return hip_fail(e, "merge kernel launch");
+    if ((e = sqa::launch_merge(ma, cus, s)) != hipSuccess) return hip_fail(e, "merge kernel launch");
   }
   if (ev && (e = hipEventRecord(ev[2], s)) != hipSuccess) return hip_fail(e, "hipEventRecord");
   return SQA_OK;

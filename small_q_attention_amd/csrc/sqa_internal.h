@@ -297,7 +297,30 @@ inline int seam_pages(int rows, int hkv, int head_dim, int kv_bytes) {
   return c < 1 ? 1 : (c > 32 ? 32 : c);
 }
 
+// Threads that share one of `rows` output rows in the merge kernel, of a workgroup's
+// 256. A partial row takes `chunks` threads (16 bytes each), an output row has about
+// `per_row` splits, and each thread issues U loads at once (the smallest U of 2, 4, 8
+// that covers the row; more rounds past 8). Three ways to share a row's splits:
+// - the threads of one partial row take all of the row's splits, several rows per
+//   wave and no exchange between lanes: up to 8 splits per row where the rows
+//   still come to two waves per SIMD of the device's `cus` compute units. A wave per
+//   row leaves most of its lanes without a split there and takes four times the waves
+//   (whole calls, wave per row -> this: 64 short ragged sequences, q_len 4, 58.0 ->
+//   55.9 us; 64 of 512 keys, q_len 16, 45.1 -> 36.6; 128 of up to 1K, q_len 8, 78.8 ->
+//   67.2). At half as many rows the two are even (16 of 8K, q_len 8: 87.9 and 87.4) or
+//   the wave per row is ahead (16 of up to 2K, q_len 8: 27.5 and 28.1);
+// - a wave per row (4 rows per workgroup) from 1024 rows on, wherever 8 loads per
+//   thread cover the row's splits;
+// - a workgroup of 4 waves per row below that, or where a wave would need a
+//   second round (one sequence, KV 32K, q_len 8: 128 splits per row).
+inline int merge_row_threads(long long rows, int per_row, int chunks, int cus) {
+  constexpr int kWave = 64, kSimds = 4, kWavesPerSimd = 2;
+  if (cus > 0 && per_row <= 8 && rows * chunks >= (long long)cus * kSimds * kWavesPerSimd * kWave)
+    return chunks;
+  return rows >= 1024 && per_row <= 8 * (kWave / chunks) ? kWave : 4 * kWave;
+}
+
 hipError_t launch_partial(const PartialArgs& a, hipStream_t stream);
-hipError_t launch_merge(const MergeArgs& a, hipStream_t stream);
+hipError_t launch_merge(const MergeArgs& a, int cus, hipStream_t stream);
 
 }  // namespace sqa

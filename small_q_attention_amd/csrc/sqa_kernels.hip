@@ -2550,48 +2550,28 @@ void launch_merge_u(const MergeArgs& a, int u, hipStream_t stream) {
 }
 
 template <int HD, typename E, bool BAL>
-void launch_merge_hd(const MergeArgs& a, int per_row, hipStream_t stream) {
-  // Three ways to share a row's splits, each thread issuing U loads of 16 bytes at
-  // once (the smallest U of 2, 4, 8 that covers the row; more rounds past 8):
-  // - the threads of one partial row take all of the row's splits, several rows per
-  //   wave and no exchange between lanes: up to 8 splits per row where the rows
-  //   still come to two waves per SIMD. A wave per row leaves most of its lanes
-  //   without a split there and takes four times the waves (whole calls, wave per
-  //   row -> this: 64 short ragged sequences, q_len 4, 58.0 -> 55.9 us; 64 of 512
-  //   keys, q_len 16, 45.1 -> 36.6; 128 of up to 1K, q_len 8, 78.8 -> 67.2). At
-  //   half as many rows the two are even (16 of 8K, q_len 8: 87.9 and 87.4) or the
-  //   wave per row is ahead (16 of up to 2K, q_len 8: 27.5 and 28.1);
-  // - a wave per row (4 rows per workgroup) from 1024 rows on, wherever 8 loads per
-  //   thread cover the row's splits;
-  // - a workgroup of 4 waves per row below that, or where a wave would need a
-  //   second round (one sequence, KV 32K, q_len 8: 128 splits per row).
+void launch_merge_hd(const MergeArgs& a, int per_row, int cus, hipStream_t stream) {
   constexpr int kChunks = HD / (E::kHalfPartials ? 8 : 4);  // threads a partial row takes
-  constexpr int kSplitsPerWave = 64 / kChunks;
-  constexpr long long kManyThreads = 256 * 4 * 2 * 64;
-  const int total = a.batch * a.q_len * a.hq;
-  if constexpr (kChunks < 64) {
-    if ((long long)total * kChunks >= kManyThreads && per_row <= 8) {
-      launch_merge_u<HD, E, kChunks, BAL>(a, per_row, stream);
-      return;
-    }
-  }
-  if (total >= 1024 && per_row <= 8 * kSplitsPerWave) {
-    const int u = (per_row + kSplitsPerWave - 1) / kSplitsPerWave;
-    launch_merge_u<HD, E, 64, BAL>(a, u, stream);
-  } else {
-    const int u = (per_row + 4 * kSplitsPerWave - 1) / (4 * kSplitsPerWave);
+  const int threads =
+      merge_row_threads((long long)a.batch * a.q_len * a.hq, per_row, kChunks, cus);
+  const int at_once = threads / kChunks;  // splits per load instruction
+  const int u = (per_row + at_once - 1) / at_once;
+  if (threads == 256)
     launch_merge_u<HD, E, 256, BAL>(a, u, stream);
-  }
+  else if (threads == 64)
+    launch_merge_u<HD, E, 64, BAL>(a, u, stream);
+  else
+    launch_merge_u<HD, E, kChunks, BAL>(a, u, stream);
 }
 
 template <typename E, bool BAL>
-void launch_merge_as(const MergeArgs& a, int per_row, hipStream_t stream) {
+void launch_merge_as(const MergeArgs& a, int per_row, int cus, hipStream_t stream) {
   if (a.head_dim == 64)
-    launch_merge_hd<64, E, BAL>(a, per_row, stream);
+    launch_merge_hd<64, E, BAL>(a, per_row, cus, stream);
   else if (a.head_dim == 256)
-    launch_merge_hd<256, E, BAL>(a, per_row, stream);
+    launch_merge_hd<256, E, BAL>(a, per_row, cus, stream);
   else
-    launch_merge_hd<128, E, BAL>(a, per_row, stream);
+    launch_merge_hd<128, E, BAL>(a, per_row, cus, stream);
 }
 
 template <bool BAL>
@@ -2611,11 +2591,11 @@ void launch_partial_plan(const PartialArgs& a, const LaunchShape& sh, dim3 grid,
 }
 
 template <bool BAL>
-void launch_merge_plan(const MergeArgs& a, int per_row, hipStream_t stream) {
+void launch_merge_plan(const MergeArgs& a, int per_row, int cus, hipStream_t stream) {
   if (a.bf16)
-    launch_merge_as<ElemBF16, BAL>(a, per_row, stream);
+    launch_merge_as<ElemBF16, BAL>(a, per_row, cus, stream);
   else
-    launch_merge_as<ElemF16, BAL>(a, per_row, stream);
+    launch_merge_as<ElemF16, BAL>(a, per_row, cus, stream);
 }
 
 }  // namespace
@@ -2637,7 +2617,7 @@ hipError_t launch_partial(const PartialArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_merge(const MergeArgs& a, hipStream_t stream) {
+hipError_t launch_merge(const MergeArgs& a, int cus, hipStream_t stream) {
   // Splits per sequence, for the choice of merge variant: a fixed plan's
   // num_splits; the balanced plan's count per sequence is known only on the
   // device: the batch average, items / batch. It depends on the slot count
@@ -2650,9 +2630,9 @@ hipError_t launch_merge(const MergeArgs& a, hipStream_t stream) {
   const int per_row = is_balanced(a.pages_per_split) ? (items + a.batch - 1) / a.batch
                                                      : a.num_splits;
   if (is_balanced(a.pages_per_split))
-    launch_merge_plan<true>(a, per_row, stream);
+    launch_merge_plan<true>(a, per_row, cus, stream);
   else
-    launch_merge_plan<false>(a, per_row, stream);
+    launch_merge_plan<false>(a, per_row, cus, stream);
   return hipGetLastError();
 }
 
