@@ -26,8 +26,8 @@
 //     8*(l%16)+0..7 (four full 256-byte rows per instruction) and regroups
 //     them with one byte permute per half pair: output block mb covers dims
 //     d = 8*m + mb, m = 0..15.
-// Rows beyond q_len*group (q_len*group not a multiple of 16) carry zero Q and
-// are never stored. The figures above are for head dim 128; the kernels are
+// Rows beyond q_len*group (q_len*group not a multiple of 16) carry some row's Q
+// (zeros in the 8-wave kernel) and are never stored. The figures above are for head dim 128; the kernels are
 // also built for 64 and 256 (HD), where the per-lane counts scale with HD
 // (Dims<HD>) and a ring slot holds a page of HD-wide rows, and at head dim 64
 // a wave takes two kv heads (HPW = 2; a workgroup then serves 8 kv heads):
@@ -1388,10 +1388,11 @@ struct StagedBits {
 // non-temporal.
 // The two kinds of plan are instantiations of their own (BAL: balanced), here and in
 // the merge kernel: a call of a few pages runs almost every instruction for the
-// first time, and the way to its first load led around the other plan's code (per
-// call, one kernel for both -> each its own: one sequence of 1K keys, q_len 2, 10.2
-// -> 9.3 us; of 8K, q_len 4, 13.85 -> 13.2, q_len 8 17.7 -> 16.7; of 4K, q_len 16,
-// 18.7 -> 17.3; long calls +-0.3%).
+// first time, and the way to its first load led around the other plan's code (the
+// GPU's part of a call, back to back, one kernel for both -> each its own: one
+// sequence of 1K keys, q_len 2, 10.2 -> 9.3 us, where the whole call is bounded by the
+// host's part, 12.4; of 8K, q_len 4, 13.85 -> 13.2, q_len 8 17.7 -> 16.7; of 4K, q_len
+// 16, in the 8-wave kernel, 18.7 -> 17.3; long calls +-0.3%).
 // The page ring runs through the pieces of an item: the next piece's first pages
 // are requested in this one's last turn and its Q and mask words as soon as this
 // one begins, so a sequence end costs the epilogue (about 1 us) and not a drained

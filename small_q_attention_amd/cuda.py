@@ -230,9 +230,10 @@ def _traced_op(query, key_cache, value_cache, block_tables, seq_lens,
     split plan at run time from the tensors' shapes, so a dynamic batch size needs
     no recompilation. A measured ``max_seq_len`` (-1: ``seq_lens.max().item()``, a
     host sync) plans over the whole block-table row instead, so the graph never
-    synchronises; its splits differ from the measured plan's only past the
-    sequences' ends (empty), which changes the merge's summation order, not which
-    keys count."""
+    synchronises. With a chunk size the splits then differ from the measured plan's
+    only past the sequences' ends (empty); the automatic plan of one sequence is
+    sized for the row instead of the length. Either changes how the sums round, not
+    which keys count."""
     import torch
 
     from . import _op  # noqa: F401  (registers the ops)

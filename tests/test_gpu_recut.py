@@ -139,3 +139,52 @@ def test_a_promised_length_does_not_change_the_bits(q_len, lens, width):
         ns, pps = _lib.plan_splits(0, len(lens), q_len, 32, 8, 128, promise, width, 0)
         own = _lib.workspace_bytes(len(lens), q_len, 32, 8, 128, ns, pps)
         assert torch.equal(_call(dev, ns, pps, own + (64 << 20)), plain), promise
+
+
+@pytest.mark.parametrize("lens,width,cut", [
+    ([1500] * 8, 94, True), ([1500] * 8, 200, False),  # splits of 6 pages; 14 would be needed
+    ([1100] * 5, 300, True), ([1100] * 5, 301, False),  # of 12; 14
+    ([300] * 40, 24, True), ([300] * 40, 60, False),   # of 8; 20
+])
+def test_which_batches_are_cut_at_their_starts(lens, width, cut):
+    """A balanced plan leaves its (first slot, count) table in the workspace; one that is
+    cut runs as a fixed plan and leaves that part alone. 256 compute units (two head
+    groups of the 8 kv heads share them)."""
+    if _lib.load().sqa_device_cu_count(0) != 256:
+        pytest.skip("the widths are those of 256 compute units")
+    q, k, v, bt, sl = inputs.make_inputs(
+        inputs.Case(batch=len(lens), q_len=2, seq_lens=lens, seed=2700))
+    wide = torch.zeros(len(lens), width, dtype=torch.int32)
+    wide[:, :bt.shape[1]] = bt
+    dev = tuple(t.cuda() for t in (q, k, v, wide, sl))
+    ns, pps = _lib.plan_splits(0, len(lens), 2, 32, 8, 128, max(lens), width, 0)
+    assert pps < 0
+    nbytes = _lib.workspace_bytes(len(lens), 2, 32, 8, 128, ns, pps)
+    ws = torch.full((nbytes // 4,), float("nan"), device="cuda")
+    out = torch.empty_like(dev[0])
+    _lib.launch(*dev, out, ws, ns, pps, torch.cuda.current_stream().cuda_stream)
+    table = ws[ns * 8 * 8 * (128 + 2):][:2 * len(lens)]
+    assert torch.isnan(table).all().item() == cut
+    assert torch.isnan(table).any().item() == cut
+    assert_parity(out, attention_c64(q, k, v, bt, sl, 16, 8), label=f"width {width}")
+
+
+def test_a_chunked_plan_over_a_table_past_two_to_the_31_entries():
+    """Three rows of 2**30 pages each (12 GiB, of which a few pages are written): the third
+    row starts at entry 2**31."""
+    width = 1 << 30
+    free, _ = torch.cuda.mem_get_info()
+    if free < 20 << 30:
+        pytest.skip("needs 20 GiB of device memory")
+    lens = [700, 90, 660]
+    q, k, v, bt, sl = inputs.make_inputs(
+        inputs.Case(batch=3, q_len=4, seq_lens=lens, seed=2800))
+    table = torch.empty(3, width, dtype=torch.int32, device="cuda")
+    table[:, :64].zero_()
+    table[:, :bt.shape[1]] = bt.cuda()
+    dev = (q.cuda(), k.cuda(), v.cuda(), table, sl.cuda())
+    own = _lib.workspace_bytes(3, 4, 32, 8, 128, 6, 8)
+    out = _call(dev, 6, 8, own + (64 << 20))
+    del dev, table
+    torch.cuda.empty_cache()
+    assert_parity(out, attention_c64(q, k, v, bt, sl, 16, 8), label="wide table")
